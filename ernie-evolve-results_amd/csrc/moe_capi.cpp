@@ -146,7 +146,8 @@ static int check_route(const void* x, const void* w, int w_dtype, int T, int H, 
 // block histograms as well).
 static bool route_is_fused(int T, int H, int E, int w_dtype, const moe_route_cfg* cfg) {
   return T > 0 && w_dtype == MOE_DTYPE_BF16 &&
-         moe::route_fused_supported(E, H, cfg->scoring, cfg->n_group);
+         moe::route_fused_supported(E, H, cfg->scoring, cfg->n_group) &&
+         !moe::router_wk_use(T, H, E, false);
 }
 
 // Whether route_launch takes the small-E kernel (E = 8 or 16 with bf16
@@ -221,6 +222,17 @@ static int route_launch(const void* x, const void* w, int w_dtype, const float* 
                                             cfg->topk_group, cfg->route_scale, cfg->norm_min,
                                             logits, topk_ids, topk_w, counts, blockcnt, ws, s),
                     "route_fused");
+  if (moe::router_wk_use(T, H, E, w_dtype == MOE_DTYPE_FP32)) {
+    const int rc = launched(moe::launch_router_wk((const __bf16*)x, w, w_dtype == MOE_DTYPE_FP32,
+                                                  T, H, E, logits, s),
+                            "router_wk");
+    if (rc) return rc;
+    return launched(moe::launch_topk(logits, 1, bias, T, E, k, cfg->scoring, cfg->renormalize,
+                                     cfg->n_group, cfg->topk_group, cfg->route_scale,
+                                     cfg->norm_min, nullptr, topk_ids, topk_w, counts, blockcnt,
+                                     s),
+                    "topk");
+  }
   const int N = w_dtype == MOE_DTYPE_FP32 ? 2 * E : E;
   const int ksplit = moe::router_gemm_ksplit(T, H, N);
   const int parts = (N / E) * ksplit;
@@ -260,6 +272,10 @@ int moe_router_gemm(const void* x, const void* w, int T, int H, int E, float* lo
   if (!supported_e(E)) return fail(MOE_ERR_UNSUPPORTED, "E=%d not in {8,...,256}", E);
   if (!aligned16(x) || !aligned16(w)) return fail(MOE_ERR_ALIGNMENT, "x/w not 16-byte aligned");
   if (T == 0) return ok();
+  if (moe::router_wk_use(T, H, E, false))
+    return launched(moe::launch_router_wk((const __bf16*)x, w, false, T, H, E, logits,
+                                          (hipStream_t)stream),
+                    "router_wk");
   return launched(moe::launch_router_gemm((const __bf16*)x, (const __bf16*)w, T, H, E, 1, logits,
                                           (hipStream_t)stream),
                   "router_gemm");

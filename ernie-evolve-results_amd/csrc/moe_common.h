@@ -52,6 +52,17 @@ hipError_t launch_wsplit(const float* w, __bf16* wpk, int E, int H, hipStream_t 
 hipError_t launch_router_gemm(const __bf16* x, const __bf16* w, int T, int H, int N,
                               int ksplit, float* out, hipStream_t s);
 int router_gemm_ksplit(int T, int H, int N);
+// The router GEMM with K split over the waves of a block (router_wk.hip), for
+// batches too small to fill the chip with whole-K tiles: whether (T, H, E) takes
+// it, and its launch (w bf16 [E, H], or with wf32 fp32 [E, H] split hi/lo in the
+// kernel).  out: the logits [T, E], no partial sums.
+bool router_wk_use(int T, int H, int E, bool wf32);
+hipError_t launch_router_gemm_128x64(const __bf16* x, const void* w, int T, int H, int N,
+                                     float* out, hipStream_t s);
+hipError_t launch_router_gemm_128x128(const __bf16* x, const void* w, int T, int H, int N,
+                                      float* out, hipStream_t s);
+hipError_t launch_router_wk(const __bf16* x, const void* w, bool wf32, int T, int H, int E,
+                            float* out, hipStream_t s);
 // blockcnt (or NULL; needs topk_block_hist_supported): also the permute's raw
 // block histograms [E, dispatch_blocks(T*k)], every entry written.
 hipError_t launch_topk(const float* logits, int nparts, const float* bias, int T, int E, int k,

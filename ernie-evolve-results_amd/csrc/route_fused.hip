@@ -1,5 +1,7 @@
 // Stages 1+2 in one kernel at E = 256 and E = 128: router GEMM + scoring +
-// top-k + histogram, with the logits tile kept on chip.
+// top-k + histogram, with the logits tile kept on chip.  For batches whose
+// tiles fill more than half the chip (T > 16384 and T > 10240; smaller ones
+// take router_wk.hip and the scoring kernel, router_wk_use).
 //
 // Replaces the reference's cublasGemmEx (K:4327-4339) followed by
 // topk_kernel (K:1829-1920), which writes the [T,E] fp32 logits to HBM and

@@ -212,4 +212,14 @@ hipError_t launch_router_gemm(const __bf16* x, const __bf16* w, int T, int H, in
   return launch_dma<32, 16, 4, 2, 1>(x, w, T, H, N, ksplit, out, s);
 }
 
+// Whole-K tiles for the batches router_wk.hip gives them (w bf16).
+hipError_t launch_router_gemm_128x64(const __bf16* x, const void* w, int T, int H, int N,
+                                     float* out, hipStream_t s) {
+  return launch_dma<128, 64, 6, 4, 2>(x, (const __bf16*)w, T, H, N, 1, out, s);
+}
+hipError_t launch_router_gemm_128x128(const __bf16* x, const void* w, int T, int H, int N,
+                                      float* out, hipStream_t s) {
+  return launch_dma<128, 128, 5, 2, 4>(x, (const __bf16*)w, T, H, N, 1, out, s);
+}
+
 }  // namespace moe

@@ -1,0 +1,299 @@
+// Stage 1 for batches too small to fill the chip with whole-K tiles: the
+// router GEMM with K split over the waves of a block.
+//
+// The fused kernel (route_fused.hip) gives a block 128 (64) tokens and all E
+// experts, so a batch of T tokens runs on T / 128 of the 256 CUs and each of
+// those streams the whole weight: at E = 256, H = 7168 the route took 91 us
+// for any T from 1 to 4096.  Such a call is bound by what one CU can load
+// (a DMA stream of 128-byte rows moves about 90 GB/s per CU here), so the
+// tile is chosen for the fewest operand bytes per CU: BM tokens x BN experts
+// with BM + BN as small as leaves at most one block per CU.  A block's four
+// waves split K, each streaming its quarter through its own LDS ring by
+// the gfx950 buffer_load ... lds DMA (8 rows of 128 bytes per instruction,
+// XOR-swizzled 16-byte chunks); only the wave that fills a ring reads it, so
+// the K loop has no barrier, and the ring is as deep as the LDS allows.
+// The partial tiles meet in LDS and are added in K order.
+// The blocks of one row tile are 8 apart in the grid: one XCD, whose L2 serves
+// the row tile's x to all of them.
+//
+// Measured (MI355X; route = this GEMM + the scoring kernel, graph replay, us,
+// the path it replaced first): E = 256, H = 7168: T = 4 91 / 13, 128 91 / 15,
+// 1024 92 / 22, 4096 98 / 44, 8192 99 / 67, 16384 105 / 102; E = 128,
+// H = 2048: T = 128 19 / 9.5, 4096 20 / 15; E = 64, H = 4096: T = 128
+// 11.5 / 8.9.  GEMM alone at E = 256, H = 7168, T = 16: fragments loaded
+// straight into registers (16 rows x 64 bytes per load instruction, so every
+// four lanes touch four lines) 15.4 us, this ring 6.5; 8 waves x 2 stages 7.0,
+// 4 waves x 3 stages 7.7.
+//
+// An fp32 weight (WF32) comes into the ring as fp32 and each lane splits its 8
+// k into hi = bf16(w) and lo = bf16(w - hi) (the reference's wsplit_kernel,
+// K:1786-1824); a logit is (sum of hi) + (sum of lo), each in K order.  That
+// saves the split's launch, its [2E, H] copy and the partial sums: E = 64,
+// H = 8192 T = 128 20.5 / 13.5, T = 3000 32.7 / 28.9; E = 256, H = 1024
+// T = 128 20.7 / 11.5.
+#include "moe_common.h"
+
+namespace moe {
+
+namespace wk {
+// word 3 of a gfx9 raw buffer resource (32-bit data format, no swizzle)
+constexpr int kRsrcW3 = 0x00020000;
+// an offset past every resource here: such a load writes zeros and moves nothing
+constexpr int kPast = 0x7f000000;
+__device__ __forceinline__ int swz(int r) { return (r >> 1) & 7; }
+// 16 bytes per lane into LDS (1 KB per wave instruction)
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, char* l, int voff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)l, 16, voff,
+                                           0, 0, 0);
+}
+}  // namespace wk
+
+// BM tokens x BN experts per block, NW waves with NS-stage rings; E % BN == 0.
+// mtiles = ceil(T / BM); the grid rounds the row tiles up to a multiple of 8.
+template <int BM, int BN, int NW, int NS, bool WF32>
+__global__ __launch_bounds__(64 * NW) void router_wk_kernel(const __bf16* __restrict__ x,
+                                                            const void* __restrict__ w, int T,
+                                                            int H, int E, int mtiles,
+                                                            float* __restrict__ out) {
+  using namespace wk;
+  constexpr int FM = BM / 16, FN = BN / 16;
+  constexpr int WB = WF32 ? 4 : 2;       // bytes per weight element
+  constexpr int NP = WF32 ? 2 : 1;       // hi and lo products
+  constexpr int LD = BN + 4;             // row stride of a partial tile in LDS (floats)
+  constexpr int WROWB = 64 * WB;         // weight bytes per row and stage
+  constexpr int XB = BM * 128, STAGE_B = XB + BN * WROWB;
+  constexpr int NQX = XB / 1024, NQ = STAGE_B / 1024;
+  constexpr int RING_B = NW * NS * STAGE_B, PART_B = NW * BM * LD * 4;
+  __shared__ __attribute__((aligned(1024))) char lds[RING_B > PART_B ? RING_B : PART_B];
+  static_assert(sizeof(lds) <= 160 * 1024, "LDS");
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nt_n = E / BN;
+  const int j8 = (int)blockIdx.x >> 3;
+  const int nt = j8 % nt_n;
+  const int mt = (j8 / nt_n) * 8 + ((int)blockIdx.x & 7);
+  if (mt >= mtiles) return;
+  const long long m0 = (long long)mt * BM;
+  const int rows = T - m0 < BM ? (int)(T - m0) : BM;
+  const int n0 = nt * BN;
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(x + m0 * H), (short)0, rows * H * 2, kRsrcW3);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)((const char*)w + (long long)n0 * H * WB), (short)0, BN * H * WB, kRsrcW3);
+
+  // this wave's K steps of 64: [u0, u1)
+  const int U = H / 64;
+  const int u0 = wave * U / NW, u1 = (wave + 1) * U / NW, n = u1 - u0;
+  char* const ring = lds + wave * NS * STAGE_B;
+  // Per-lane source of each DMA instruction of a stage: 16-byte chunk p of row r
+  // goes to physical chunk p ^ swz(r), an fp32 weight row's 32-byte chunk c to
+  // c ^ (r & 7).  Rows past T and steps past u1 lie past the resource (zeros),
+  // so every step issues the same loads and the waits below are constants.
+  int voff[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    if (q < NQX) {
+      const int r = q * 8 + lane / 8;
+      voff[q] = r * H * 2 + u0 * 128 + ((lane % 8) ^ swz(r)) * 16;
+    } else if (!WF32) {
+      const int r = (q - NQX) * 8 + lane / 8;
+      voff[q] = r * H * 2 + u0 * 128 + ((lane % 8) ^ swz(r)) * 16;
+    } else {
+      const int r = (q - NQX) * 4 + lane / 16;  // 16 lanes of 16 B: 8 chunks of 32 B
+      voff[q] = r * H * 4 + u0 * 256 + ((((lane % 16) >> 1) ^ (r & 7)) * 32) + (lane & 1) * 16;
+    }
+  }
+  auto issue = [&](int u, int st) {
+    const int kx = u < n ? u * 128 : kPast;
+    const int kw = u < n ? u * WROWB : kPast;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      char* dst = ring + st * STAGE_B + q * 1024;
+      if (q < NQX) dma16(rx, dst, voff[q] + kx);
+      else dma16(rw, dst, voff[q] + kw);
+    }
+  };
+
+  f32x4 acc[NP][FM][FN];
+#pragma unroll
+  for (int p = 0; p < NP; ++p)
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[p][i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int st = 0; st < NS - 1; ++st) issue(st, st);
+  const int fr = lane & 15, fc = lane >> 4;
+  int slot = 0;
+  for (int u = 0; u < n; ++u) {
+    // stage u landed once at most the NS-2 later stages are outstanding; the
+    // slot refilled now held step u-1, whose reads its MFMAs have consumed
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * NQ) : "memory");
+    const int nslot = slot == 0 ? NS - 1 : slot - 1;
+    issue(u + NS - 1, nslot);
+    const char* sb = ring + slot * STAGE_B;
+    slot = slot == NS - 1 ? 0 : slot + 1;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const int c = kk * 4 + fc;
+      bf16x8 av[FM];
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const int r = i * 16 + fr;
+        av[i] = *reinterpret_cast<const bf16x8*>(sb + r * 128 + ((c ^ swz(r)) * 16));
+      }
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        const int r = j * 16 + fr;
+        bf16x8 bh, bl;
+        if constexpr (WF32) {
+          const f32x4* pv = reinterpret_cast<const f32x4*>(sb + XB + r * WROWB + (c ^ (r & 7)) * 32);
+          const f32x4 v0 = pv[0], v1 = pv[1];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float v = e < 4 ? v0[e & 3] : v1[e & 3];
+            bh[e] = (__bf16)v;
+            bl[e] = (__bf16)(v - (float)bh[e]);
+          }
+        } else {
+          bh = *reinterpret_cast<const bf16x8*>(sb + XB + r * 128 + ((c ^ swz(r)) * 16));
+        }
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+          acc[0][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], bh, acc[0][i][j], 0, 0, 0);
+          if constexpr (WF32)
+            acc[1][i][j] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], bl, acc[1][i][j], 0, 0, 0);
+        }
+      }
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the loads past u1 have landed
+  __syncthreads();  // every ring is read: the partial tiles may overwrite them
+  float* const part = reinterpret_cast<float*>(lds);
+
+  constexpr int NT = 64 * NW, NV = BM * BN / 4;  // 16-byte pieces of the tile
+  constexpr int PER = (NV + NT - 1) / NT;
+  f32x4 sum[PER];
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    if (p > 0) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          part[(wave * BM + i * 16 + fc * 4 + r) * LD + j * 16 + fr] = acc[p][i][j][r];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      const int idx = threadIdx.x + q * NT;
+      if (NV % NT != 0 && idx >= NV) continue;
+      const int row = idx / (BN / 4), c4 = idx % (BN / 4);
+      const float* s = part + row * LD + c4 * 4;
+      f32x4 v = *reinterpret_cast<const f32x4*>(s);
+#pragma unroll
+      for (int g = 1; g < NW; ++g) v += *reinterpret_cast<const f32x4*>(s + g * BM * LD);
+      sum[q] = p == 0 ? v : sum[q] + v;
+    }
+  }
+  const bool vec = ((uintptr_t)out & 15u) == 0;  // moe_router_gemm takes 4-byte aligned logits
+#pragma unroll
+  for (int q = 0; q < PER; ++q) {
+    const int idx = threadIdx.x + q * NT;
+    if (NV % NT != 0 && idx >= NV) continue;
+    const int row = idx / (BN / 4), c4 = idx % (BN / 4);
+    if (row >= rows) continue;
+    float* o = out + (m0 + row) * E + n0 + c4 * 4;
+    if (vec) {
+      *reinterpret_cast<f32x4*>(o) = sum[q];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = sum[q][e];
+    }
+  }
+}
+
+template <int BM, int BN, int NW, int NS, bool WF32>
+static hipError_t launch_wk(const __bf16* x, const void* w, int T, int H, int E, float* out,
+                            hipStream_t s) {
+  const int mt = (T + BM - 1) / BM;
+  const dim3 grid((unsigned)((mt + 7) / 8 * 8 * (E / BN)));
+  hipLaunchKernelGGL((router_wk_kernel<BM, BN, NW, NS, WF32>), grid, dim3(64 * NW), 0, s, x, w, T,
+                     H, E, mt, out);
+  return hipGetLastError();
+}
+
+namespace wk {
+struct Tile {
+  int bm, bn;
+  hipError_t (*launch)(const __bf16*, const void*, int, int, int, float*, hipStream_t);
+};
+// The last two are the shared-ring kernel of router_gemm.hip (K in order, all of a
+// block's waves on one tile), for batches of several rounds.
+const Tile kTiles[] = {
+    {16, 16, launch_wk<16, 16, 4, 4, false>}, {32, 16, launch_wk<32, 16, 4, 3, false>},
+    {16, 32, launch_wk<16, 32, 4, 3, false>}, {48, 16, launch_wk<48, 16, 4, 3, false>},
+    {32, 32, launch_wk<32, 32, 4, 3, false>}, {48, 32, launch_wk<48, 32, 4, 3, false>},
+    {64, 32, launch_wk<64, 32, 4, 3, false>}, {32, 64, launch_wk<32, 64, 4, 3, false>},
+    {48, 64, launch_wk<48, 64, 4, 2, false>}, {64, 64, launch_wk<64, 64, 4, 2, false>},
+    {80, 64, launch_wk<80, 64, 4, 2, false>}, {128, 64, launch_router_gemm_128x64},
+    {128, 128, launch_router_gemm_128x128}};
+const Tile kTilesF32[] = {{16, 16, launch_wk<16, 16, 8, 2, true>},
+                          {32, 16, launch_wk<32, 16, 8, 2, true>},
+                          {48, 16, launch_wk<48, 16, 8, 2, true>}};
+constexpr int kCUs = 256;
+
+// The tile of the least operand bytes per CU: rounds of blocks x operand rows
+// per block (an fp32 weight row counts twice).  Measured over T = 1 .. 16384 at
+// E = 32 .. 256, H = 512 .. 8192 it picks the fastest tile or one within 5% of it.
+static const Tile* pick(int T, int E, bool wf32) {
+  const Tile* t = wf32 ? kTilesF32 : kTiles;
+  const int n = (int)(wf32 ? sizeof(kTilesF32) : sizeof(kTiles)) / (int)sizeof(Tile);
+  const Tile* best = nullptr;
+  long long least = 0;
+  for (int i = 0; i < n; ++i) {
+    if (E % t[i].bn) continue;
+    const long long blocks = (long long)((T + t[i].bm - 1) / t[i].bm) * (E / t[i].bn);
+    const long long c = (blocks + kCUs - 1) / kCUs * (t[i].bm + (wf32 ? 2 : 1) * t[i].bn);
+    if (!best || c < least) {
+      best = t + i;
+      least = c;
+    }
+  }
+  return best;
+}
+}  // namespace wk
+
+// Where it takes over (route times in us, the other path / this one):
+//   E = 256, H = 7168 and E = 128, H = 2048 (the fused kernel's shapes): while
+//     the fused kernel's tiles fill under ~2/3 of the CUs: T = 16384 105 / 102,
+//     24000 116 / 188; T = 10000 22.4 / 21.6, 12000 24.8 / 29.6.
+//   elsewhere, against K split over blocks with the partial sums added by the
+//     scoring kernel: that path moves fewer operand bytes (larger tiles) but
+//     writes and reads the partials, so it wins for long rows and many tokens:
+//     E = 256, H = 4096 T = 12000 74 / 64, 16384 73 / 70, 32768 118 / 167;
+//     E = 64, H = 8192 T = 2500 20.4 / 19.0, 3000 23.0 / 25.9; E = 128,
+//     H = 7168 T = 3000 28.0 / 27.8, 4096 30.4 / 33.1 -- and at E = 128 from
+//     T = 10000 on the 128 x 128 tile beats its 64-row tiles (72 / 56).
+//   fp32 weights: E = 64, H = 8192 T = 3000 32.7 / 28.9, 4096 34.9 / 42.0;
+//     E = 256, H = 4096 T = 700 30 / 19, 4096 42 / 61; E = 32, H = 4096
+//     T = 6000 22.9 / 20.0, 8192 27.9 / 29.1.
+bool router_wk_use(int T, int H, int E, bool wf32) {
+  if (T < 1 || E < 32 || H % 64 != 0 || H > 32768) return false;
+  if (wf32) return (long long)T * E <= (H <= 4096 ? 229376 : 196608);
+  if (E == 256 && H == 7168) return T <= 16384;
+  if (E == 128 && H == 2048) return T <= 10240;
+  if (E == 128 && T > 8192) return true;
+  return H <= 4096 ? T <= 12288 : (long long)T * H <= 2560ll * 8192;
+}
+
+hipError_t launch_router_wk(const __bf16* x, const void* w, bool wf32, int T, int H, int E,
+                            float* out, hipStream_t s) {
+  const wk::Tile* t = wk::pick(T, E, wf32);
+  return t ? t->launch(x, w, T, H, E, out, s) : hipErrorInvalidValue;
+}
+
+}  // namespace moe

@@ -79,7 +79,7 @@ const char* moe_last_error_string(void);
  *     weights (hi and lo halves) or a K split (ksplit > 1, chosen when the
  *     row x expert tiles alone leave the chip's 256 CUs idle, e.g. small T):
  *     [T, parts*E] fp32 partial sums.
- *   - E = 256, H = 7168 or E = 128, H = 2048 with bf16 weights: the router
+ *   - E = 256, H = 7168 or E = 128, H = 2048 with bf16 weights: for large T the
  *     GEMM and the scoring run as one kernel that reads a fragment-major copy
  *     of the weight, E*H*2 bytes (3.5 MiB / 512 KiB), rewritten by every call.
  * E = 8 or 16 with bf16 weights and H % 256 == 0 (the Mixtral shape): zero;
@@ -109,8 +109,9 @@ int moe_topk(const float* logits, const float* bias, int T, int E, int k,
  * into bf16 hi/lo on the device (wsplit_kernel K:1786-1824) so the bf16 GEMM
  * yields fp32-accurate logits.  logits [T,E] fp32 (the reference's
  * router_logits output), counts may be NULL.  With bf16 weights at E = 256,
- * H = 7168 or E = 128, H = 2048 the GEMM and the scoring are one kernel
- * (unless a group-limited rule's groups are not multiples of 32 experts at
+ * H = 7168 (T > 16384) or E = 128, H = 2048 (T > 10240) the GEMM and the
+ * scoring are one kernel; smaller batches split K over the waves of a block
+ * instead (unless a group-limited rule's groups are not multiples of 32 experts at
  * E = 256, 16 at E = 128: then the two-kernel path, same results). */
 int moe_route(const void* x, const void* w, int w_dtype, const float* bias, int T, int H,
               int E, int k, const moe_route_cfg* cfg, float* logits, int32_t* topk_ids,

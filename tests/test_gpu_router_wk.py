@@ -1,0 +1,112 @@
+"""The router GEMM with K split over the waves of a block (csrc/router_wk.hip):
+logits against the float64 product, at token counts on both sides of its tiles
+(16 to 128 tokens) and of the rule that picks it, for bf16 and fp32 weights.
+
+Bound: a sum of H products in fp32 in any order is within H * 2^-24 * sum |x||w|;
+an fp32 weight's hi/lo split adds 2^-16 of that sum (hi + lo keeps 16 bits of w)."""
+import pytest
+import torch
+
+import moe_route as M
+from moe_route.configs import RouteCfg
+
+pytestmark = pytest.mark.gpu
+
+# (E, H): H = 64 leaves three of the four waves without a K step, 576 splits
+# unevenly, the rest are the fused kernel's shapes and ordinary ones
+SHAPES = [(32, 64), (64, 576), (128, 2048), (256, 7168), (256, 1024)]
+TOKENS = [1, 15, 17, 48, 257, 513, 1025, 3073, 4133, 6001]
+
+
+def inputs(T, H, E, seed, dev):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    x = torch.randn(T, H, generator=g, device=dev).bfloat16()
+    return x, torch.randn(E, H, generator=g, device=dev) * 0.02
+
+
+def assert_logits(got, x, w, split):
+    ref = x.double() @ w.double().t()
+    mag = x.double().abs() @ w.double().abs().t()
+    bound = (2 * x.shape[1] * 2.0 ** -24 + (2.0 ** -16 if split else 0.0)) * mag
+    assert bool(((got.double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("E,H", SHAPES)
+@pytest.mark.parametrize("T", TOKENS)
+@pytest.mark.parametrize("fp32", [False, True])
+def test_logits(cuda, E, H, T, fp32):
+    print("router_wk E=%d H=%d T=%d fp32=%d" % (E, H, T, fp32), flush=True)
+    x, w = inputs(T, H, E, T + E, cuda)
+    w = w if fp32 else w.bfloat16()
+    k = min(8, E)
+    logits, ids, wts, counts = M.route(x, w, None, k, RouteCfg())
+    assert_logits(logits, x, w, fp32)
+    # the scoring on the same logits, and the histogram
+    i2, w2, c2 = M.topk(logits, None, k, RouteCfg())
+    assert torch.equal(ids, i2) and torch.equal(wts, w2) and torch.equal(counts, c2)
+    if not fp32:
+        assert_logits(M.router_gemm(x, w), x, w, False)
+
+
+def test_unaligned_logits(cuda):
+    """moe_router_gemm takes logits at any 4-byte address."""
+    T, H, E = 33, 1024, 64
+    x, w = inputs(T, H, E, 5, cuda)
+    w = w.bfloat16()
+    buf = torch.full((T * E + 2,), -7.0, device=cuda)
+    out = buf[1:-1]
+    M._check(M.lib().moe_router_gemm(M._ptr(x), M._ptr(w), T, H, E, M._ptr(out), M._stream(x)))
+    assert torch.equal(out.view(T, E), M.router_gemm(x, w))
+    assert float(buf[0]) == -7.0 and float(buf[-1]) == -7.0
+
+
+@pytest.mark.parametrize("E,H,T", [(256, 7168, 16384), (256, 7168, 16385), (256, 7168, 16500),
+                                   (128, 2048, 10240), (128, 2048, 10241), (128, 2048, 10370)])
+@pytest.mark.parametrize("rule", ["sigmoid_group", "softmax", "softmax_bias"])
+def test_fused_kernel_either_side_of_the_rule(cuda, E, H, T, rule):
+    """At the fused kernel's shapes: the last batch that goes to this GEMM, the
+    first that goes to the fused kernel, and one that ends inside a fused tile;
+    logits, ids, weights and counts equal the standalone GEMM and scoring."""
+    cfg = {"sigmoid_group": RouteCfg(M.SCORING_SIGMOID_GROUP, True, E // 32, 4, 2.5),
+           "softmax": RouteCfg(M.SCORING_SOFTMAX, True),
+           "softmax_bias": RouteCfg(M.SCORING_SOFTMAX_BIAS, True, norm_min=1e-6)}[rule]
+    k = 8 if T % 2 else 5
+    x, w = inputs(T, H, E, T, cuda)
+    w = w.bfloat16()
+    bias = torch.randn(E, device=cuda, generator=torch.Generator(device=cuda).manual_seed(T)) * 0.1
+    logits, ids, wts, counts = M.route(x, w, bias, k, cfg)
+    assert torch.equal(logits, M.router_gemm(x, w))
+    i2, w2, c2 = M.topk(logits, bias, k, cfg)
+    assert torch.equal(ids, i2) and torch.equal(wts, w2) and torch.equal(counts, c2)
+
+
+@pytest.mark.parametrize("topk_group", [1, 2, 3, 4, 6, 8])
+@pytest.mark.parametrize("k", [8, 6])
+def test_fused_kernel_ties(cuda, topk_group, k):
+    """The fused kernel's epilogue ranks two tokens per lane group (with at most 4
+    kept groups in compacted rounds): the same choice as the scoring kernel where
+    scores tie exactly inside and across groups (rows and bias repeat every 37)."""
+    E, H, T = 256, 7168, 16391
+    cfg = RouteCfg(M.SCORING_SIGMOID_GROUP, True, 8, topk_group, 2.5)
+    x, w = inputs(T, H, 37, 100 + topk_group, cuda)
+    at = torch.arange(E, device=cuda) % 37
+    w = w.bfloat16()[at].contiguous()
+    bias = (torch.arange(37, device=cuda) * 0.37).sin()[at].contiguous()
+    logits, ids, wts, counts = M.route(x, w, bias, k, cfg)
+    assert torch.equal(logits[:, 0], logits[:, 37])
+    i2, w2, c2 = M.topk(logits, bias, k, cfg)
+    assert torch.equal(ids, i2) and torch.equal(wts, w2) and torch.equal(counts, c2)
+
+
+@pytest.mark.parametrize("E,H,T,k", [(256, 7168, 16391, 8), (256, 7168, 16391, 2),
+                                     (128, 2048, 10241, 8), (128, 2048, 10241, 4)])
+def test_fused_kernel_block_histograms(cuda, E, H, T, k):
+    """The fused kernel's histogram handoff in the one-call step: the same
+    permutation as from the ids alone."""
+    x, w = inputs(T, H, E, T + k, cuda)
+    w = w.bfloat16()
+    plan = M.MoePlan(T, H, E, k, RouteCfg(), cuda)
+    plan.route_permute(x, w, None, index_only=True)
+    p = M.permute(x, plan.topk_ids, E, index_only=True)
+    for name in ("row_token", "pair_row", "offsets", "counts"):
+        assert torch.equal(getattr(plan, name), p[name]), name
