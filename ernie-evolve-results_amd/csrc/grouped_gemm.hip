@@ -17,30 +17,56 @@
 // sized by the bound sum ceil(m_g / BM) <= ceil(M / BM) + G; blocks past the
 // last tile return at once.
 //
-// Tiles: 256 rows x 256 weight rows (128 x 512 for groups of at most 128
-// rows on average), 128-byte K steps (64 bf16 or 128 int8 elements), staged
-// in LDS by the gfx950 global_load_lds DMA into a 2-stage ring with an
-// XOR-swizzled 16-byte chunk layout, v_mfma_f32_16x16x32_bf16 or
-// v_mfma_i32_16x16x64_i8 accumulators (bf16 / int8 A: 8 waves of 64 x 128
-// with a software-pipelined K loop; fp8 A: 16 waves of 64 x 64, plain loop).
+// Tiles: 256 rows x 256 weight rows, 128-byte K steps (64 bf16 or 128 int8
+// elements), staged in LDS by the gfx950 global_load_lds DMA in an XOR-swizzled
+// 16-byte chunk layout, v_mfma_f32_16x16x32_bf16 or v_mfma_i32_16x16x64_i8.
+// Eight waves in two groups of four (one wave of each per SIMD); a wave owns 64
+// rows of each 128-row half of the tile and 32 weight rows of each half.
+//
+// K loop.  A K step is two half steps (the two row halves); each wave does, per
+// half step, a load part (12 fragment reads, 4 DMA instructions) and 32 MFMAs,
+// with a barrier after each, and the second group runs one barrier behind the
+// first: while one group's MFMAs hold the matrix pipes the other reads
+// fragments and issues loads.  The operand tile is recycled in quarters: the
+// rows read in one half step are refilled in the next (every wave has waited for
+// its reads before the barrier in between), for the step after next, so a load
+// has three half steps to land and 96 of the 128 KB are in flight or in use.
+// One 256 x 256 tile per CU at 85% MFMA busy (counters, K = 8192; the previous
+// loop, both waves of a SIMD in step and the whole stage refilled at once: 71%).
+// Measured, dense (TFLOP/s or TOP/s, previous loop first): 16384 x 16384 x 8192
+// bf16 1292 / 1489, SwiGLU 1337 / 1501, int8 2623 / 2854; 65536 x 8192 x 3584 bf16
+// 1310 / 1451, int8 2268 / 2455.  The rest is the clock: 1.48 GHz at this load.
+// The routed experts (64 experts, H = 8192, Ni = 3584, top-8, us): gate+up T = 16
+// 1229 / 1136, 1024 1794 / 1313, 2048 2398 / 2073; the 128 x 512 tiles that small
+// groups had are slower everywhere but the int8 down projection at T = 16 ..
+// 768 (332 / 356 at T = 64).  Tried and slower: four half steps of 16 MFMAs (5%
+// instead of 13% gained), s_setprio around the MFMAs (-1%), the DMA issued
+// between the MFMAs (-8%), the closing barrier 2 .. 12 MFMAs early (-8 .. -12%),
+// 32x32x16 MFMAs (-13%).
+//
+// fp8 A: the DMA brings each wave's own 16 rows of e4m3fn bytes, and half a K step
+// before they are read the wave writes them once as bf16(q * s) into the A tile
+// (one tile is enough: its halves are refilled as above).  1708 / 1533 us at
+// T = 1024, 5004 / 4341 at T = 4096 against a dequantisation pass with its own
+// barrier in every step.
+//
 // Block ids are remapped so that each XCD runs a contiguous range of logical
 // tiles, and inside a group the tiles go in 4 x 8 (row x column) super-tiles:
 // the blocks running together on one XCD share A and weight slices in L2.
 //
-// swiglu interleaves the two weights at 16-row granularity inside the B
-// tile (rows 16f..16f+15 come from wg for even f, from wu for odd f), so the
-// gate and up accumulators of the same output columns sit in one wave and
-// the epilogue forms h without an exchange.  A tile then covers half its
-// weight rows in output columns.
+// swiglu: the first half of the weight rows is the gate, the second the up
+// projection of the same 128 output columns, so both accumulators of a column
+// sit in one lane and the epilogue forms h without an exchange.
 //
 // Identity shortcut (the reference's ident_a / ident_m): a group whose row
 // count equals ident_m takes its A rows from ident_a (row i of the group =
 // row i of ident_a) instead of a.
 #include "moe_common.h"
+#include <utility>
 
 namespace moe {
 
-constexpr int kGgBN = 256;  // narrowest tile: weight rows per tile (tile shape: template parameters)
+constexpr int kGgBM = 256, kGgBN = 256;  // rows and weight rows of a tile
 
 // One workgroup of 1024 threads: inclusive scan of per-group tile counts.
 __global__ __launch_bounds__(1024) void gg_plan_kernel(const int* __restrict__ offs, int G, int M,
@@ -148,65 +174,29 @@ __device__ __forceinline__ typename AccOf<I8>::type mfma_step(bf16x8 a, bf16x8 b
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// 32-bit LDS address of a __shared__ location, for inline-asm LDS reads.
-__device__ __forceinline__ unsigned lds_addr(const void* p) {
-  return (unsigned)(uintptr_t)((__attribute__((address_space(3))) const char*)p);
-}
-
 // The A operand's row map (bf16 and int8 A) and the row / column scales of the
 // int8 operands (unused by the bf16 and fp8 paths).
 struct GgExtra {
-  const float* a;      // int8: per row of a
+  const float* a;      // int8: per row of a; fp8: [M, K/128]
   const int* a_idx;    // NULL, or [M]: operand row r is row a_idx[r] of a (data and scale)
   const float* ident;  // [ident_m] per row of ident_a
   const float* w0;     // [G, N] per weight row of w0
   const float* w1;     // [G, N] per weight row of w1 (SwiGLU up)
 };
 
-template <bool SWIGLU, bool AFP8, int BK, int NS, int WM, int WN, bool PIPE, int BM, bool I8,
-          int BNT>
-__global__ __launch_bounds__(64 * WM * WN) void grouped_gemm_kernel(
-    const void* __restrict__ a_, const float* __restrict__ a_scales, const void* __restrict__ ident_,
-    int ident_m, const void* __restrict__ w0_, const void* __restrict__ w1_,
-    const int* __restrict__ offs, const int* __restrict__ tile_start, int G, int M, int N, int K,
-    int n_tiles, unsigned short* __restrict__ out, GgExtra i8s) {
-  // LDS rows: B (weights) BK*WEL bytes; A BK*2 bytes (bf16) or BK bytes (fp8,
-  // int8).  bf16 steps are 64 wide, int8 steps 128 wide: 128-byte rows either
-  // way.  A DMA wave instruction moves 1 KB = 1024 / row-bytes rows.
-  constexpr int BN = BNT;  // weight rows per tile
-  constexpr int WEL = I8 ? 1 : 2;  // bytes per weight element
-  constexpr int ROWB = BK * WEL, CH = ROWB / 16, RPI = 1024 / ROWB;
-  constexpr int AROWB = (AFP8 || I8) ? BK : BK * 2, ACH = AROWB / 16, ARPI = 1024 / AROWB;
-  // MFMA depth: v_mfma_f32_16x16x32_bf16 or v_mfma_i32_16x16x64_i8; both
-  // take 16 bytes per lane with the same lane -> (row, K chunk) layout.
-  constexpr int KSUB = I8 ? 64 : 32;
-  const char* const w0 = (const char*)w0_;
-  const char* const w1 = (const char*)w1_;
-  constexpr int A_BYTES = BM * AROWB, STAGE_B = A_BYTES + BN * ROWB;
-  // fp8 A: the DMA stages hold the e4m3fn bytes; each K step they are
-  // dequantised once, cooperatively, into one bf16 tile (BM x BK) that the
-  // fragment reads use.
-  constexpr int DQ_BYTES = AFP8 ? BM * BK * 2 : 0;
-  constexpr int NW = WM * WN, NT = 64 * NW;
-  constexpr int A_INST = BM / ARPI, B_INST = BN / RPI, PER_WAVE = (A_INST + B_INST) / NW;
-  constexpr int WTM = BM / WM, WTN = BN / WN, FM = WTM / 16, FN = WTN / 16;
-  static_assert(I8 ? BK == 128 : (BK == 32 || BK == 64), "K step of one or two MFMA depths");
-  static_assert(!(I8 && AFP8), "int8 and fp8 A are separate paths");
-  static_assert((A_INST + B_INST) % NW == 0, "every wave issues the same number of loads");
-  static_assert(!AFP8 || BK == 64, "fp8 A: one 128-wide scale block spans two K steps");
-  static_assert(!AFP8 || (BM * ACH) % NT == 0, "fp8 A: whole 16-byte chunks per thread per K step");
-  static_assert(!SWIGLU || FN % 2 == 0, "swiglu: gate/up fragment pairs inside one wave");
-  static_assert(!PIPE || (!AFP8 && ROWB == 128 && NS == 2 &&
-                          ((BM == 256 && BN == 256 && WM == 4 && WN == 2) ||
-                           (BM == 128 && BN == 512 && WM == 2 && WN == 4))),
-                "pipelined loop: bf16 / int8 A, 2 stages of 128-byte rows, 8 waves of 64 x 128: "
-                "256 x 256 or 128 x 512 tiles");
-  __shared__ __attribute__((aligned(1024))) char lds[NS * STAGE_B + DQ_BYTES];
-  char* const dq = lds + NS * STAGE_B;
-  const char* a = (const char*)a_;
-  const char* ident_a = (const char*)ident_;
-  constexpr int AEL = (AFP8 || I8) ? 1 : 2;  // bytes per A element
-
+// The tile of block blockIdx.x: false if the block has none.  BM rows per tile.
+struct GgTile {
+  int g;      // group
+  int gs;     // its first row
+  int r0;     // first row of the tile
+  int rlast;  // last row of the group
+  int nt;     // column tile
+  bool ident; // A rows from ident_a
+};
+template <int BM>
+__device__ __forceinline__ bool gg_tile(const int* __restrict__ offs,
+                                        const int* __restrict__ tile_start, int G, int M,
+                                        int n_tiles, int ident_m, GgTile& out) {
   // XCD-aware order: hardware block b runs on XCD b % 8.  The grid is sized
   // by a bound on the tile count; the real count nreal is known here, and the
   // logical tiles [x*r, (x+1)*r), r = ceil(nreal / 8), all run on XCD x, so
@@ -235,9 +225,9 @@ __global__ __launch_bounds__(64 * WM * WN) void grouped_gemm_kernel(
   total_rt = __builtin_amdgcn_readfirstlane(total_rt);  // wave-uniform: keep it in an SGPR
   const unsigned nreal = (unsigned)total_rt * (unsigned)n_tiles;
   const unsigned r = (nreal + 7u) >> 3;
-  if ((b >> 3) >= r) return;
+  if ((b >> 3) >= r) return false;
   const unsigned l = (b & 7u) * r + (b >> 3);
-  if (l >= nreal) return;
+  if (l >= nreal) return false;
   const int lt = (int)(l / (unsigned)n_tiles);
   // group g of row tile lt: gstart <= lt < gstart + mtg (the first group whose
   // inclusive tile count exceeds lt; groups without tiles never qualify)
@@ -292,365 +282,405 @@ __global__ __launch_bounds__(64 * WM * WN) void grouped_gemm_kernel(
   const int ge = min(max(offs[g], 0), M);
   const int r0 = gs + mt_local * BM;               // first row of the tile
   const int rlast = ge - 1;                        // last row of the group
-  const bool ident = ident_m > 0 && ge - gs == ident_m;
-
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wave / WN, wn = wave % WN;
-  // A wave whose rows all lie past the group (the last, partial row tile of a
-  // group) still issues its share of the DMA and joins every barrier, but
-  // skips its fragment reads and MFMAs: its results are never stored.
-  const bool live = r0 + wm * WTM <= rlast;
-  // logical 16-byte chunk c of an LDS row r sits at c ^ swz(r): the 16 rows
-  // of one fragment read fall on distinct bank groups
-  auto swz = [](int r, int ch) { return ch == 8 ? (r >> 1) & 7 : (r >> 2) & 3; };
-  const long long wbase = (long long)g * N * K * WEL;  // bytes
-
-  // DMA sources (bytes) and the byte advance per K step of each instruction
-  const char* src[PER_WAVE];
-  int kstep[PER_WAVE];
-#pragma unroll
-  for (int q = 0; q < PER_WAVE; ++q) {
-    const int gi = wave * PER_WAVE + q;
-    if (gi < A_INST) {
-      const int r = gi * ARPI + lane / ACH, p = lane % ACH;
-      const int row = min(r0 + r, rlast);  // rows past the group are loaded, never stored
-      const int arow_i = (!ident && i8s.a_idx) ? i8s.a_idx[row] : row;
-      const char* arow = ident ? ident_a + (long long)(row - gs) * K * AEL
-                               : a + (long long)arow_i * K * AEL;
-      src[q] = arow + (p ^ swz(r, ACH)) * 16;
-      kstep[q] = BK * AEL;
-    } else {
-      const int r = (gi - A_INST) * RPI + lane / CH, p = lane % CH;
-      int wrow;
-      const char* wsrc = w0;
-      if (SWIGLU) {
-        const int f = r >> 4;
-        wrow = nt * (BN / 2) + (f >> 1) * 16 + (r & 15);
-        if (f & 1) wsrc = w1;
-      } else {
-        wrow = nt * BN + r;
-      }
-      wrow = min(wrow, N - 1);
-      src[q] = wsrc + wbase + (long long)wrow * K * WEL + (p ^ swz(r, CH)) * 16;
-      kstep[q] = BK * WEL;
-    }
-  }
-  auto issue = [&](int kt, int st) {
-#pragma unroll
-    for (int q = 0; q < PER_WAVE; ++q) {
-      auto* dst = (__attribute__((address_space(3))) void*)(lds + st * STAGE_B +
-                                                            (wave * PER_WAVE + q) * 1024);
-      __builtin_amdgcn_global_load_lds((const void*)(src[q] + (long long)kt * kstep[q]), dst, 16,
-                                       0, 0);
-    }
-  };
-
-  // fp8: every K step thread t dequantises the 16-byte chunks t, t + NT, ...
-  // (chunk q: tile row q / ACH, 16-byte column q % ACH); it keeps each of
-  // its rows' scales for the current 128-wide K block and the next block's,
-  // loaded one block ahead.
-  const int fr = lane & 15, fc = lane >> 4;
-  const int nsb = K / 128;
-  constexpr int DQ_PER = AFP8 ? BM * ACH / NT : 1;
-  float sc[DQ_PER], scn[DQ_PER];
-  int dq_row[DQ_PER];
-#pragma unroll
-  for (int u = 0; u < DQ_PER; ++u) {
-    dq_row[u] = min(r0 + (int)(threadIdx.x + u * NT) / ACH, rlast) * nsb;
-    sc[u] = AFP8 ? a_scales[dq_row[u]] : 0.0f;
-    scn[u] = AFP8 && nsb > 1 ? a_scales[dq_row[u] + 1] : 0.0f;
-  }
-
-  using AccV = typename AccOf<I8>::type;
-  AccV acc[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = AccV{0, 0, 0, 0};
-
-  const int KT = K / BK;
-  if constexpr (PIPE) {
-    // Software-pipelined K loop, two 128-byte-row stages, each K step in two
-    // halves (kk = 0, 1) with their own fragment registers F0 / F1.  The
-    // MFMAs of a half are interleaved with the LDS reads of the next half's
-    // fragments (one read after every second MFMA) and, in the kk = 1 half,
-    // with the DMA of the stage after next (one instruction after every
-    // fourth MFMA), so neither the LDS queue nor the DMA issue holds the
-    // matrix pipe.  Step s:
-    //   wait F0 (stage s, kk 0); MFMA(F0) + reads F1 (stage s, kk 1);
-    //   wait F1 and stage s+1's DMA (this wave); barrier (every wave: stage
-    //   s+1 landed, the reads of stage s done);
-    //   MFMA(F1) + reads F0 (stage s+1, kk 0) + DMA of stage s+2 into stage
-    //   s's buffer.
-    // Each accumulator sees K steps ascending, kk 0 then 1: bit-identical to
-    // the plain loop.
-    const unsigned l0 = lds_addr(lds);
-    unsigned abase[2][2], bbase[2][2];  // [stage][kk]: fragment 0; fragment i / j at +i*2048 / +j*2048
-#pragma unroll
-    for (int st = 0; st < 2; ++st)
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        const unsigned c = (unsigned)(((kk * 4 + fc) ^ swz(fr, CH)) * 16);
-        abase[st][kk] = l0 + st * STAGE_B + (wm * WTM + fr) * AROWB + c;
-        bbase[st][kk] = l0 + st * STAGE_B + A_BYTES + (wn * WTN + fr) * ROWB + c;
-      }
-    bf16x8 a0[FM], b0[FN], a1[FM], b1[FN];
-    // One 16-byte LDS fragment read issued as an instruction the compiler does
-    // not track: the loop places its own lgkmcnt waits, so the reads stay in
-    // flight across the MFMAs they are interleaved with.
-    auto read_one = [&](bf16x8& dst, unsigned addr) {
-      asm volatile("ds_read_b128 %0, %1" : "=v"(dst) : "v"(addr));
-    };
-    auto dma_one = [&](int q, int kt, int st) {
-      auto* dst = (__attribute__((address_space(3))) void*)(lds + st * STAGE_B +
-                                                            (wave * PER_WAVE + q) * 1024);
-      __builtin_amdgcn_global_load_lds((const void*)(src[q] + (long long)kt * kstep[q]), dst, 16,
-                                       0, 0);
-    };
-    constexpr int kReads = FM + FN;
-    // DMA instruction q follows MFMA q * kDs + kDs / 2
-    constexpr int kDs = FM * FN >= 4 * PER_WAVE ? 4 : 2;
-    static_assert(2 * kReads <= FM * FN && kDs * PER_WAVE <= FM * FN,
-                  "the reads and the DMA fit between the MFMAs of a half step");
-    // MFMAs on (av, bv); reads into (ra, rb) from (rab, rbb) when rd; DMA of
-    // stage dkt into buffer dst when dkt >= 0
-    auto half = [&](bf16x8 (&av)[FM], bf16x8 (&bv)[FN], bf16x8 (&ra)[FM], bf16x8 (&rb)[FN],
-                    unsigned rab, unsigned rbb, bool rd, int dkt, int dst) {
-#pragma unroll
-      for (int t = 0; t < FM * FN; ++t) {
-        acc[t / FN][t % FN] = mfma_step<I8>(av[t / FN], bv[t % FN], acc[t / FN][t % FN]);
-        if ((t & 1) && (t >> 1) < kReads && rd) {
-          const int r = t >> 1;
-          if (r < FM) read_one(ra[r], rab + r * 2048);
-          else read_one(rb[r - FM], rbb + (r - FM) * 2048);
-        }
-        if (t % kDs == kDs / 2 && t / kDs < PER_WAVE && dkt >= 0) dma_one(t / kDs, dkt, dst);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    };
-    issue(0, 0);
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    if (KT > 1) issue(1, 1);
-    if (!live) {
-      // DMA and barriers only, in the same order as the live loop below
-      for (int k2 = 0; k2 < KT; ++k2) {
-        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-        if (k2 + 2 < KT) issue(k2 + 2, k2 & 1);
-      }
-    } else {
-#pragma unroll
-      for (int r = 0; r < FM; ++r) read_one(a0[r], abase[0][0] + r * 2048);
-#pragma unroll
-      for (int r = 0; r < FN; ++r) read_one(b0[r], bbase[0][0] + r * 2048);
-      for (int kt = 0; kt < KT; kt += 2) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int k2 = kt + u;  // stage k2 lives in buffer u
-          if (k2 < KT) {
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // F0 of stage k2
-            __builtin_amdgcn_sched_barrier(0);
-            half(a0, b0, a1, b1, abase[u][1], bbase[u][1], true, -1, 0);
-            // F1 landed (this wave's reads of stage k2 are done) and stage
-            // k2+1's DMA landed; the barrier makes both true for every wave
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            __builtin_amdgcn_sched_barrier(0);
-            half(a1, b1, a0, b0, abase[u ^ 1][0], bbase[u ^ 1][0], k2 + 1 < KT,
-                 k2 + 2 < KT ? k2 + 2 : -1, u);
-          }
-        }
-      }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  } else {
-  #pragma unroll
-    for (int st = 0; st < NS - 1; ++st)
-      if (st < KT) issue(st, st);
-    for (int kt = 0; kt < KT; ++kt) {
-      // this wave's stage kt landed once at most the NS-2 later stages are
-      // outstanding; the barrier then publishes every wave's DMA and retires
-      // all reads of the buffer reloaded next
-      if (kt + NS - 2 < KT)
-        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 2) * PER_WAVE) : "memory");
-      else
-        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-      if (kt + NS - 1 < KT) issue(kt + NS - 1, (kt + NS - 1) % NS);
-      const char* sb = lds + (kt % NS) * STAGE_B;
-      if (AFP8) {
-        const bool nb = kt > 0 && (kt & 1) == 0;  // a new 128-wide scale block starts
-  #pragma unroll
-        for (int u = 0; u < DQ_PER; ++u) {
-          if (nb) {
-            sc[u] = scn[u];
-            scn[u] = (kt >> 1) + 1 < nsb ? a_scales[dq_row[u] + (kt >> 1) + 1] : 0.0f;
-          }
-          const int q = threadIdx.x + u * NT, r = q / ACH, c = q % ACH;
-          const u32x4 raw = *reinterpret_cast<const u32x4*>(sb + r * AROWB + ((c ^ swz(r, ACH)) * 16));
-          bf16x8 lo8, hi8;
-          dequant16(raw, sc[u], lo8, hi8);
-          *reinterpret_cast<bf16x8*>(dq + r * ROWB + (((2 * c) ^ swz(r, CH)) * 16)) = lo8;
-          *reinterpret_cast<bf16x8*>(dq + r * ROWB + (((2 * c + 1) ^ swz(r, CH)) * 16)) = hi8;
-        }
-        // the bf16 tile is complete for every wave (its previous contents were
-        // retired by the barrier at the top of this step)
-        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-        __builtin_amdgcn_s_barrier();
-      }
-      if (!live) continue;
-  #pragma unroll
-      for (int kk = 0; kk < BK / KSUB; ++kk) {
-        bf16x8 bv[FN];
-  #pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          const int r = wn * WTN + j * 16 + fr, c = kk * 4 + fc;
-          bv[j] = *reinterpret_cast<const bf16x8*>(sb + A_BYTES + r * ROWB + ((c ^ swz(r, CH)) * 16));
-        }
-        bf16x8 av[FM];
-  #pragma unroll
-        for (int i = 0; i < FM; ++i) {
-          const int r = wm * WTM + i * 16 + fr, c = kk * 4 + fc;
-          av[i] = AFP8 ? *reinterpret_cast<const bf16x8*>(dq + r * ROWB + ((c ^ swz(r, CH)) * 16))
-                       : *reinterpret_cast<const bf16x8*>(sb + r * AROWB + ((c ^ swz(r, ACH)) * 16));
-        }
-  #pragma unroll
-        for (int i = 0; i < FM; ++i)
-  #pragma unroll
-          for (int j = 0; j < FN; ++j)
-            acc[i][j] = mfma_step<I8>(av[i], bv[j], acc[i][j]);
-      }
-    }
-  }
-
-  // Epilogue: lane holds rows (lane>>4)*4 + r, column lane & 15 of each 16x16 tile.
-  // int8: value = float(acc) * (row scale * column scale), in that order.  All
-  // scales are loaded before the first store (a load issued after a store
-  // would wait for it: both count in vmcnt).
-  constexpr int OUTC = SWIGLU ? BN / 2 : BN;  // output columns of a tile
-  float cs0[FN], cs1[FN], rsc[FM][4];
-#pragma unroll
-  for (int j = 0; j < FN; ++j) {
-    cs0[j] = cs1[j] = 1.0f;
-    if constexpr (I8) {
-      const int col = SWIGLU ? nt * (BN / 2) + (wn * FN + (j & ~1)) / 2 * 16 + (lane & 15)
-                             : nt * BN + wn * WTN + j * 16 + (lane & 15);
-      if (col < N) {
-        cs0[j] = i8s.w0[(long long)g * N + col];
-        if (SWIGLU) cs1[j] = i8s.w1[(long long)g * N + col];
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      rsc[i][r] = 1.0f;
-      if constexpr (I8) {
-        const int row = min(r0 + wm * WTM + i * 16 + (lane >> 4) * 4 + r, rlast);
-        rsc[i][r] = ident ? i8s.ident[row - gs] : i8s.a[i8s.a_idx ? i8s.a_idx[row] : row];
-      }
-    }
-  // output value of accumulator (i, j, r); SwiGLU pairs j (gate) with j + 1 (up)
-  auto value = [&](int i, int j, int r) -> float {
-    if (SWIGLU) {
-      float gv, uv;
-      if constexpr (I8) {
-        gv = (float)acc[i][j][r] * (rsc[i][r] * cs0[j]);
-        uv = (float)acc[i][j + 1][r] * (rsc[i][r] * cs1[j]);
-      } else {
-        gv = acc[i][j][r];
-        uv = acc[i][j + 1][r];
-      }
-      return swiglu(gv, uv);
-    }
-    if constexpr (I8) return (float)acc[i][j][r] * (rsc[i][r] * cs0[j]);
-    else return acc[i][j][r];
-  };
-  constexpr int JSTEP = SWIGLU ? 2 : 1;
-  const int ldo = N;
-  if ((N & 7) == 0) {
-    // Stage the bf16 tile in LDS (the operand buffers are idle once every wave is
-    // past its last fragment read), then write whole 16-byte chunks of output
-    // rows.  LDS row = OUTC bf16; 16-byte chunk c of tile row rl sits at
-    // c ^ (2 * ((rl >> 2) & 3)), so the four row groups one ds_write covers
-    // land in distinct banks.
-    static_assert(BM * OUTC * 2 <= (int)sizeof(lds), "output tile fits in the LDS");
-    constexpr int RCH = OUTC / 8;
-    unsigned short* ct = reinterpret_cast<unsigned short*>(lds);
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int rl = wm * WTM + i * 16 + (lane >> 4) * 4 + r;
-        const int sw = 2 * ((rl >> 2) & 3);
-#pragma unroll
-        for (int j = 0; j < FN; j += JSTEP) {
-          const int cl = (SWIGLU ? (wn * FN + j) / 2 * 16 : wn * WTN + j * 16) + (lane & 15);
-          ct[rl * OUTC + (((cl >> 3) ^ sw) << 3) + (cl & 7)] = (unsigned short)f2bf(value(i, j, r));
-        }
-      }
-    __syncthreads();
-    const int c0 = nt * OUTC;
-    for (int q = threadIdx.x; q < BM * RCH; q += NT) {
-      const int rl = q / RCH, c = q % RCH;
-      const int row = r0 + rl, col = c0 + c * 8;
-      if (row > rlast || col >= N) continue;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(ct + rl * OUTC +
-                                                      ((c ^ (2 * ((rl >> 2) & 3))) << 3));
-      *reinterpret_cast<u32x4*>(out + (long long)row * ldo + col) = v;
-    }
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = r0 + wm * WTM + i * 16 + (lane >> 4) * 4 + r;
-      if (row > rlast) continue;
-      unsigned short* orow = out + (long long)row * ldo;
-#pragma unroll
-      for (int j = 0; j < FN; j += JSTEP) {
-        const int col = SWIGLU ? nt * (BN / 2) + (wn * FN + j) / 2 * 16 + (lane & 15)
-                               : nt * BN + wn * WTN + j * 16 + (lane & 15);
-        if (col < N) orow[col] = (unsigned short)f2bf(value(i, j, r));
-      }
-    }
+  out = GgTile{g, gs, r0, rlast, nt, ident_m > 0 && ge - gs == ident_m};
+  return true;
 }
 
 int grouped_gemm_n_tiles(int N, bool swiglu) {
   const int per = swiglu ? kGgBN / 2 : kGgBN;
   return (N + per - 1) / per;
 }
-template <int BNT>
-static int n_tiles_of(int N, bool swiglu) {
-  const int per = swiglu ? BNT / 2 : BNT;
-  return (N + per - 1) / per;
+enum GgType { kBf16, kInt8, kFp8 };  // A; the weights are bf16, int8, bf16
+
+namespace gg {
+constexpr int kHalf = 128 * 128;       // bytes of a half operand tile: 128 rows of 128 bytes
+constexpr int kRaw = 128 * 64;         // fp8: the same half as e4m3fn bytes
+// LDS map.  bf16 / int8: two K steps of B0, A0, B1, A1.  fp8: two K steps of
+// B0, B1, one bf16 A tile, two K steps of raw A halves, the row scales.
+template <GgType TY> __device__ constexpr int b_at(int buf, int y) {
+  return TY == kFp8 ? (buf * 2 + y) * kHalf : (buf * 4 + 2 * y) * kHalf;
+}
+template <GgType TY> __device__ constexpr int a_at(int buf, int x) {
+  return TY == kFp8 ? (4 + x) * kHalf : (buf * 4 + 2 * x + 1) * kHalf;
+}
+__device__ constexpr int raw_at(int buf, int x) { return 6 * kHalf + (buf * 2 + x) * kRaw; }
+__device__ constexpr int sc_at(int buf, int x) { return 8 * kHalf + (buf * 2 + x) * 2048; }
+template <GgType TY> constexpr int kLds = TY == kFp8 ? 8 * kHalf + 8192 : 8 * kHalf;
+
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+__device__ __forceinline__ void dma16(const char* src, char* dst) {
+  __builtin_amdgcn_global_load_lds((const void*)src,
+                                   (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+__device__ __forceinline__ void dma4(const char* src, char* dst) {
+  __builtin_amdgcn_global_load_lds((const void*)src,
+                                   (__attribute__((address_space(3))) void*)dst, 4, 0, 0);
+}
+}  // namespace gg
+
+template <bool SWIGLU, GgType TY>
+__global__ __launch_bounds__(512) void grouped_gemm_kernel(
+    const char* __restrict__ a, const char* __restrict__ ident_a, int ident_m,
+    const char* __restrict__ w0, const char* __restrict__ w1, const int* __restrict__ offs,
+    const int* __restrict__ tile_start, int G, int M, int N, int K, int n_tiles,
+    unsigned short* __restrict__ out, GgExtra ex) {
+  using namespace gg;
+  constexpr bool I8 = TY == kInt8, F8 = TY == kFp8;
+  constexpr int EL = I8 ? 1 : 2;       // bytes per weight element
+  constexpr int BM = kGgBM;
+  __shared__ __attribute__((aligned(1024))) char lds[kLds<TY>];
+  GgTile tile;
+  if (!gg_tile<BM>(offs, tile_start, G, M, n_tiles, ident_m, tile)) return;
+  // wave-uniform: in SGPRs
+  const int g = __builtin_amdgcn_readfirstlane(tile.g), gs = __builtin_amdgcn_readfirstlane(tile.gs);
+  const int r0 = __builtin_amdgcn_readfirstlane(tile.r0);
+  const int rlast = __builtin_amdgcn_readfirstlane(tile.rlast);
+  const int nt = __builtin_amdgcn_readfirstlane(tile.nt);
+  const bool ident = tile.ident;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 2, wn = wave & 3;
+  const int fr = lane & 15, fc = lane >> 4;
+  auto swz = [](int r) { return (r >> 1) & 7; };
+  const long long rowb = (long long)K * EL;
+
+  // DMA sources, advanced a K step by every issue.  Rows past the group and
+  // weight rows past N are loaded (clamped), never stored.
+  // B half y, instruction q of this wave: rows (wave*2 + q)*8 .. +8 of the half
+  const char* bsrc[2][2];
+#pragma unroll
+  for (int y = 0; y < 2; ++y)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int r = (wave * 2 + q) * 8 + lane / 8, c = (lane & 7) ^ swz(r);
+      const int wrow = SWIGLU ? nt * 128 + r : nt * 256 + y * 128 + r;
+      bsrc[y][q] = (SWIGLU && y ? w1 : w0) + ((long long)g * N + min(wrow, N - 1)) * rowb + c * 16;
+    }
+  // A half x: as B.  fp8: one instruction of 16 rows x 64 bytes, wave*16 .. +16, in
+  // lane order (only this wave reads it), and the index of the lane's row scale
+  // from the tile's first (fewer than 2^31 scales in all)
+  constexpr int NA = F8 ? 1 : 2;
+  const char* asrc[2][NA];
+  unsigned sidx[2];
+  const float* ssrc[2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int q = 0; q < NA; ++q) {
+      const int r = F8 ? wave * 16 + lane / 4 : (wave * 2 + q) * 8 + lane / 8;
+      const int c = F8 ? lane & 3 : (lane & 7) ^ swz(r);
+      const int row = min(r0 + x * 128 + r, rlast);
+      if constexpr (F8) {
+        asrc[x][q] = a + (long long)row * K + c * 16;
+        ssrc[x] = ex.a + (long long)r0 * (K / 128);
+        sidx[x] = (unsigned)((row - r0) * (K / 128));
+      } else {
+        const int arow = (!ident && ex.a_idx) ? ex.a_idx[row] : row;
+        asrc[x][q] = (ident ? ident_a + (long long)(row - gs) * rowb : a + (long long)arow * rowb) +
+                     c * 16;
+        ssrc[x] = nullptr;
+        sidx[x] = 0;
+      }
+    }
+  auto issue_b = [&](int y, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      dma16(bsrc[y][q], lds + b_at<TY>(buf, y) + (wave * 2 + q) * 1024);
+      bsrc[y][q] += 128;
+    }
+  };
+  auto issue_a = [&](int x, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < NA; ++q) {
+      dma16(asrc[x][q], lds + (F8 ? raw_at(buf, x) : a_at<TY>(buf, x)) + (wave * NA + q) * 1024);
+      asrc[x][q] += F8 ? 64 : 128;
+    }
+  };
+  auto issue_s = [&](int x, int sbuf) __attribute__((always_inline)) {
+    dma4((const char*)(ssrc[x] + sidx[x]), lds + sc_at(sbuf, x) + wave * 256);
+    ssrc[x] += 1;
+  };
+  // fp8: this wave's 16 rows of raw half x -> bf16(q * s) in the A tile.  Each
+  // element is converted once per block, half a K step before it is read.
+  auto convert = [&](int x, int buf, int sbuf) __attribute__((always_inline)) {
+    if (r0 + x * 128 + wave * 16 > rlast) return;  // all past the group: never stored
+    const float sc = *reinterpret_cast<const float*>(lds + sc_at(sbuf, x) + wave * 256 + lane * 4);
+    const u32x4 raw =
+        *reinterpret_cast<const u32x4*>(lds + raw_at(buf, x) + wave * 1024 + lane * 16);
+    bf16x8 lo8, hi8;
+    dequant16(raw, sc, lo8, hi8);
+    const int r = wave * 16 + lane / 4, c = 2 * (lane & 3);
+    char* d = lds + a_at<TY>(0, x) + r * 128;
+    *reinterpret_cast<bf16x8*>(d + ((c ^ swz(r)) * 16)) = lo8;
+    *reinterpret_cast<bf16x8*>(d + (((c + 1) ^ swz(r)) * 16)) = hi8;
+  };
+
+  using AccV = typename AccOf<I8>::type;
+  AccV acc[2][2][4][2];  // [A half][B half][16-row block][16-column block]
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[x][y][i][j] = AccV{0, 0, 0, 0};
+  bf16x8 fa[2][4], fb0[2][2][2], fb1[2][2];  // [kk][i]; B0: [step parity][kk][j]; B1: [kk][j]
+  // fragment addresses: this wave's rows of a half, chunk kk*4 + fc
+  int aoff[2], boff[2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+    const int c = ((kk * 4 + fc) ^ swz(fr)) * 16;
+    aoff[kk] = (wm * 64 + fr) * 128 + c;
+    boff[kk] = (wn * 32 + fr) * 128 + c;
+  }
+  auto read_a = [&](int x, int buf) __attribute__((always_inline)) {
+    const char* p = lds + a_at<TY>(buf, x);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        fa[kk][i] = *reinterpret_cast<const bf16x8*>(p + aoff[kk] + i * 2048);
+  };
+  auto read_b = [&](bf16x8 (&fb)[2][2], int y, int buf) __attribute__((always_inline)) {
+    const char* p = lds + b_at<TY>(buf, y);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        fb[kk][j] = *reinterpret_cast<const bf16x8*>(p + boff[kk] + j * 2048);
+  };
+  // a wave whose rows of a half all lie past the group skips its MFMAs
+  const bool live0 = r0 + wm * 64 <= rlast, live1 = r0 + 128 + wm * 64 <= rlast;
+  // the 32 MFMAs of a half step, between two barriers
+  auto mma = [&](int x, const bf16x8 (&b0)[2][2], bool live) __attribute__((always_inline)) {
+    barrier();
+    if (live) {
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+              acc[x][y][i][j] =
+                  mfma_step<I8>(fa[kk][i], y ? fb1[kk][j] : b0[kk][j], acc[x][y][i][j]);
+    }
+    barrier();
+  };
+
+  const int KT = K * EL / 128;
+  issue_b(0, 0);
+  issue_a(0, 0);
+  if constexpr (F8) issue_s(0, 0);
+  issue_b(1, 0);
+  issue_a(1, 0);
+  if constexpr (F8) issue_s(1, 0);
+  if (KT > 1) {
+    issue_b(0, 1);
+    issue_a(0, 1);
+    issue_b(1, 1);
+    if constexpr (F8) {
+      issue_a(1, 1);
+      wait_vm<6>();  // step 0 landed
+    } else {
+      wait_vm<8>();  // B0, A0 and B1 of step 0 landed
+    }
+  } else {
+    wait_vm<2>();  // not fp8 (K % 128 == 0): all but A1
+  }
+  barrier();
+  read_b(fb0[0], 0, 0);
+  if constexpr (F8) convert(0, 0, 0);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  barrier();
+  if (wm == 1) barrier();  // half a step behind the other group from here on
+  // P: parity of the step; rem: steps after it; sb (fp8): scale buffer of the step
+  auto step = [&]<int P>(std::integral_constant<int, P>, int rem, int sb)
+                  __attribute__((always_inline)) {
+    read_a(0, P);
+    read_b(fb1, 1, P);
+    if constexpr (F8) {
+      convert(1, P, sb);
+      // per half step B0 + raw A0 or B1 + raw A1 (3 loads), in even steps a scale
+      // too: what the next half needs was issued two half steps ago
+      if (rem >= 2) {
+        issue_b(0, P);
+        issue_a(0, P);
+        if (P == 0) issue_s(0, sb ^ 1);
+        wait_vm<7>();
+      } else if (P == 0) {
+        wait_vm<3>();
+      } else {
+        wait_vm<0>();
+      }
+    } else {
+      // in flight after the loads that the next half needs (A1 of this step, B0 of
+      // the next): A0 and B1 of the next step and the two elements issued here
+      if (rem >= 2) {
+        issue_a(1, P ^ 1);
+        issue_b(0, P);
+        wait_vm<8>();
+      } else if (rem == 1) {
+        issue_a(1, P ^ 1);
+        wait_vm<6>();
+      } else {
+        wait_vm<0>();
+      }
+    }
+    mma(0, fb0[P], live0);
+    read_a(1, P);
+    read_b(fb0[P ^ 1], 0, P ^ 1);  // past the last step: not used
+    if constexpr (F8) {
+      if (rem >= 1) convert(0, P ^ 1, P == 0 ? sb : sb ^ 1);
+      if (rem >= 2) {
+        issue_b(1, P);
+        issue_a(1, P);
+        if (P == 0) issue_s(1, sb ^ 1);
+        wait_vm<P == 0 ? 8 : 6>();
+      } else {
+        wait_vm<0>();
+      }
+    } else if (rem >= 2) {
+      issue_a(0, P);
+      issue_b(1, P);
+      wait_vm<8>();
+    } else {
+      wait_vm<2>();  // rem 1: A1 of the last step may still be in flight
+    }
+    mma(1, fb0[P], live1);
+  };
+  int sb = 0;
+  for (int kt = 0; kt < KT; kt += 2) {
+    step(std::integral_constant<int, 0>{}, KT - 1 - kt, sb);
+    if (F8 || kt + 1 < KT) step(std::integral_constant<int, 1>{}, KT - 2 - kt, sb);
+    if (F8) sb ^= 1;
+  }
+  if (wm == 0) barrier();
+
+  // ---- epilogue: element e of a 16 x 16 block is row fc*4 + e, column fr.
+  // SwiGLU: B half 0 is the gate, half 1 the up product of the same columns.
+  // int8: value = float(acc) * (row scale * column scale); all scales are
+  // loaded before the first store (a load issued after a store waits for it).
+  constexpr int OUTC = SWIGLU ? 128 : 256, NY = SWIGLU ? 1 : 2;
+  auto colof = [&](int y, int j) { return y * 128 + wn * 32 + j * 16 + fr; };
+  auto rowof = [&](int x, int i, int e) { return x * 128 + wm * 64 + i * 16 + fc * 4 + e; };
+  float cs[2][2], rs[2][4][4];
+#pragma unroll
+  for (int y = 0; y < 2; ++y)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      cs[y][j] = 1.0f;
+      if constexpr (I8) {
+        const int col = nt * OUTC + colof(SWIGLU ? 0 : y, j);
+        if (col < N) cs[y][j] = (SWIGLU && y ? ex.w1 : ex.w0)[(long long)g * N + col];
+      }
+    }
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        rs[x][i][e] = 1.0f;
+        if constexpr (I8) {
+          const int row = min(r0 + rowof(x, i, e), rlast);
+          rs[x][i][e] = ident ? ex.ident[row - gs] : ex.a[ex.a_idx ? ex.a_idx[row] : row];
+        }
+      }
+  auto product = [&](int x, int y, int i, int j, int e) -> float {
+    if constexpr (I8) return (float)acc[x][y][i][j][e] * (rs[x][i][e] * cs[y][j]);
+    else return acc[x][y][i][j][e];
+  };
+  auto value = [&](int x, int y, int i, int j, int e) -> float {
+    if constexpr (SWIGLU) return swiglu(product(x, 0, i, j, e), product(x, 1, i, j, e));
+    else return product(x, y, i, j, e);
+  };
+  if ((N & 7) == 0) {
+    // the bf16 tile through LDS (16-byte chunk c of row rl at c ^ 2*((rl >> 2) & 3):
+    // the four row groups of one write land in distinct banks), then whole
+    // 16-byte chunks of output rows
+    constexpr int RCH = OUTC / 8;
+    unsigned short* ct = reinterpret_cast<unsigned short*>(lds);
+    __syncthreads();
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int rl = rowof(x, i, e), sw = 2 * ((rl >> 2) & 3);
+#pragma unroll
+          for (int y = 0; y < NY; ++y)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+              const int cl = colof(y, j);
+              ct[rl * OUTC + (((cl >> 3) ^ sw) << 3) + (cl & 7)] =
+                  (unsigned short)f2bf(value(x, y, i, j, e));
+            }
+        }
+    __syncthreads();
+    const int c0 = nt * OUTC;
+    for (int q = threadIdx.x; q < BM * RCH; q += 512) {
+      const int rl = q / RCH, c = q % RCH;
+      const int row = r0 + rl, col = c0 + c * 8;
+      if (row > rlast || col >= N) continue;
+      const u32x4 v =
+          *reinterpret_cast<const u32x4*>(ct + rl * OUTC + ((c ^ (2 * ((rl >> 2) & 3))) << 3));
+      *reinterpret_cast<u32x4*>(out + (long long)row * N + col) = v;
+    }
+    return;
+  }
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = r0 + rowof(x, i, e);
+        if (row > rlast) continue;
+#pragma unroll
+        for (int y = 0; y < NY; ++y)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const int col = nt * OUTC + colof(y, j);
+            if (col < N) out[(long long)row * N + col] = (unsigned short)f2bf(value(x, y, i, j, e));
+          }
+      }
 }
 
-template <bool AFP8, int WM, int WN, bool PIPE, int BM, int NS, bool I8 = false, int BNT = 256>
-static hipError_t launch_gg(const void* a, const float* a_scales, const void* ident_a, int ident_m,
-                            const void* w0, const void* w1, const int32_t* offs, int G, int M, int N,
-                            int K, bool swiglu, void* out, int32_t* tile_start, hipStream_t s,
-                            GgExtra i8s = GgExtra{}) {
-  constexpr int BK = I8 ? 128 : 64;  // K-step elements
-  if (G > kScanG) {  // the kernel scans up to kScanG group ends itself
-    hipLaunchKernelGGL(gg_plan_kernel, dim3(1), dim3(1024), 0, s, offs, G, M, BM, tile_start);
+template <GgType TY>
+static hipError_t launch_gg(const void* a, const void* ident_a, int ident_m, const void* w0,
+                            const void* w1, const int32_t* offs, int G, int M, int N, int K,
+                            bool swiglu, void* out, int32_t* tile_start, hipStream_t s,
+                            GgExtra ex) {
+  if (G > kScanG) {
+    hipLaunchKernelGGL(gg_plan_kernel, dim3(1), dim3(1024), 0, s, offs, G, M, kGgBM, tile_start);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   if (M == 0 || N == 0 || G == 0) return hipSuccess;
-  const int n_tiles = n_tiles_of<BNT>(N, swiglu);
-  const long long m_bound = ((long long)M + BM - 1) / BM + G;
-  long long blocks = m_bound * n_tiles;
-  blocks = (blocks + 7) / 8 * 8;
-  const dim3 grid((unsigned)blocks), blk(64 * WM * WN);
+  const int n_tiles = grouped_gemm_n_tiles(N, swiglu);
+  const long long blocks = (((long long)M + kGgBM - 1) / kGgBM + G) * n_tiles;
+  const dim3 grid((unsigned)((blocks + 7) / 8 * 8)), blk(512);
   if (swiglu)
-    hipLaunchKernelGGL((grouped_gemm_kernel<true, AFP8, BK, NS, WM, WN, PIPE, BM, I8, BNT>), grid, blk,
-                       0, s, a, a_scales, ident_a, ident_m, w0, w1, offs, tile_start, G, M, N, K,
-                       n_tiles, (unsigned short*)out, i8s);
+    hipLaunchKernelGGL((grouped_gemm_kernel<true, TY>), grid, blk, 0, s, (const char*)a,
+                       (const char*)ident_a, ident_m, (const char*)w0, (const char*)w1, offs,
+                       tile_start, G, M, N, K, n_tiles, (unsigned short*)out, ex);
   else
-    hipLaunchKernelGGL((grouped_gemm_kernel<false, AFP8, BK, NS, WM, WN, PIPE, BM, I8, BNT>), grid, blk,
-                       0, s, a, a_scales, ident_a, ident_m, w0, w0, offs, tile_start, G, M, N, K,
-                       n_tiles, (unsigned short*)out, i8s);
+    hipLaunchKernelGGL((grouped_gemm_kernel<false, TY>), grid, blk, 0, s, (const char*)a,
+                       (const char*)ident_a, ident_m, (const char*)w0, (const char*)w0, offs,
+                       tile_start, G, M, N, K, n_tiles, (unsigned short*)out, ex);
   return hipGetLastError();
 }
 
@@ -662,45 +692,22 @@ hipError_t launch_grouped_gemm(const void* a, const float* a_scales, const int32
                                const void* ident_a, int ident_m, const void* w0, const void* w1,
                                const int32_t* offs, int G, int M, int N, int K, bool swiglu,
                                void* out, int32_t* tile_start, hipStream_t s) {
-  const GgExtra ex{nullptr, a_rows, nullptr, nullptr, nullptr};
-  // fp8 A (its dequantisation pass needs a barrier inside each K step): 256-row
-  // tiles, 16 waves of 64 x 64, the plain loop.
   if (a_scales)
-    return launch_gg<true, 4, 4, false, 256, 2>(a, a_scales, ident_a, ident_m, w0, w1, offs, G, M,
-                                                N, K, swiglu, out, tile_start, s);
-  // bf16 A with at most 128 rows per group on average (e.g. T = 512 routed
-  // top-8 over 64 experts): 128 x 512 tiles, which pad a small group's last
-  // row tile less than 256 x 256; against 128 x 256 they move 40 instead of 48
-  // bytes per K step per 1024 MFMA cycles.  The pipelined loop with 8 waves of
-  // 64 x 128, as below.  run() measured (ms, 128 x 512 / 256 x 256): spread
-  // routing T = 512 (64 rows per expert) int8 4.93 / 5.04, bf16 2.50 / 2.67;
-  // T = 1571 (196 rows) int8 5.69 / 5.46, bf16 3.80 / 3.29; the harness's
-  // routing (8 groups of T rows) T = 1571 int8 2.33 / 2.15, T = 2048 bf16
-  // 3.68 / 3.20.
-  if ((long long)M <= 128ll * G)
-    return launch_gg<false, 2, 4, true, 128, 2, false, 512>(a, nullptr, ident_a, ident_m, w0, w1,
-                                                            offs, G, M, N, K, swiglu, out,
-                                                            tile_start, s, ex);
-  // bf16 A, larger groups: 256 x 256 tiles, 8 waves of 64 x 128 accumulators,
-  // the software-pipelined K loop.
-  return launch_gg<false, 4, 2, true, 256, 2>(a, nullptr, ident_a, ident_m, w0, w1, offs, G, M, N,
-                                              K, swiglu, out, tile_start, s, ex);
+    return launch_gg<kFp8>(a, ident_a, ident_m, w0, w1, offs, G, M, N, K, swiglu, out, tile_start,
+                           s, GgExtra{a_scales, nullptr, nullptr, nullptr, nullptr});
+  return launch_gg<kBf16>(a, ident_a, ident_m, w0, w1, offs, G, M, N, K, swiglu, out, tile_start,
+                          s, GgExtra{nullptr, a_rows, nullptr, nullptr, nullptr});
 }
 
-// int8 A and weights, int32 accumulation, 128-wide K steps: the same tile
-// choice as bf16 (the LDS rows are 128 bytes in both).
+// int8 A and weights, int32 accumulation, 128-wide K steps (LDS rows of 128
+// bytes as in bf16).
 hipError_t launch_grouped_gemm_i8(const void* a, const float* a_rs, const int32_t* a_rs_idx,
                                   const void* ident_a, const float* ident_rs, int ident_m,
                                   const void* w0, const float* w0s, const void* w1,
                                   const float* w1s, const int32_t* offs, int G, int M, int N, int K,
                                   bool swiglu, void* out, int32_t* tile_start, hipStream_t s) {
-  const GgExtra sc{a_rs, a_rs_idx, ident_rs, w0s, swiglu ? w1s : w0s};
-  if ((long long)M <= 128ll * G)
-    return launch_gg<false, 2, 4, true, 128, 2, true, 512>(a, nullptr, ident_a, ident_m, w0, w1,
-                                                           offs, G, M, N, K, swiglu, out,
-                                                           tile_start, s, sc);
-  return launch_gg<false, 4, 2, true, 256, 2, true>(a, nullptr, ident_a, ident_m, w0, w1, offs, G,
-                                                    M, N, K, swiglu, out, tile_start, s, sc);
+  return launch_gg<kInt8>(a, ident_a, ident_m, w0, w1, offs, G, M, N, K, swiglu, out, tile_start,
+                          s, GgExtra{a_rs, a_rs_idx, ident_rs, w0s, swiglu ? w1s : w0s});
 }
 
 }  // namespace moe

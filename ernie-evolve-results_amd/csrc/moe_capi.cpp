@@ -588,7 +588,7 @@ static int grouped_common(const void* a, const float* a_scales, const int32_t* a
   if (ws_bytes < need)
     return fail(MOE_ERR_WORKSPACE, "workspace %zu bytes < %zu required", ws_bytes, need);
   if (!aligned16(ws)) return fail(MOE_ERR_ALIGNMENT, "workspace not 16-byte aligned");
-  // row tiles are 128 or 256 rows: bound by the 128-row count
+  // row tiles are 256 rows; the bound counts 128
   const long long blocks = (((long long)M + 127) / 128 + G) *
                            moe::grouped_gemm_n_tiles(N, swiglu);
   if (blocks >= (1ll << 31)) return fail(MOE_ERR_UNSUPPORTED, "too many tiles (%lld)", blocks);
