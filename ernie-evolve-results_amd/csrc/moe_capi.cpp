@@ -385,6 +385,10 @@ static int permute_launch(const void* x, int x_dtype, const int32_t* topk_ids, i
   const bool fp8 = out_dtype == MOE_DTYPE_FP8E4M3FN;
   const int elem = x_dtype == MOE_DTYPE_BF16 ? 2 : 4;
   hipStream_t s = (hipStream_t)stream;
+  if (xg && !hist && moe::small_permute_use(T, H, k, elem, fp8))
+    return launched(moe::launch_small_permute(x, elem, fp8, topk_ids, T, H, E, k, xg, scales,
+                                              row_token, pair_row, offsets, counts, s),
+                    "small_permute");
   const int nblk = moe::dispatch_blocks((long long)T * k);
   int32_t* blockcnt = (int32_t*)ws;
   int32_t* totals = (int32_t*)((char*)ws + round256((size_t)E * nblk * 4));
@@ -515,7 +519,9 @@ int moe_route_permute(const void* x, const void* w, int w_dtype, const float* bi
   // whole permute blocks, it writes the permute's block histograms and the
   // histogram launch is skipped.  The route never writes counts here: the
   // index kernel writes them from the scanned totals.
-  const RouteHist handoff = route_block_hist(T, H, E, k, w_dtype, cfg);
+  // Few pairs: the permute counts them itself in its one launch.
+  const bool small = xg && moe::small_permute_use(T, H, k, 2, out_dtype == MOE_DTYPE_FP8E4M3FN);
+  const RouteHist handoff = small ? kHistNone : route_block_hist(T, H, E, k, w_dtype, cfg);
   void* stage = (char*)pws + moe_permute_workspace_bytes(T, E, k);
   int32_t* sub = (int32_t*)((char*)pws + moe_permute_fp8_workspace_bytes(T, H, E, k));
   int32_t* hist = handoff == kHistSub ? sub : handoff == kHistBlocks ? (int32_t*)pws : nullptr;

@@ -112,6 +112,13 @@ hipError_t launch_gather(const void* x, int elem_bytes, const int32_t* pair_row,
 hipError_t launch_gather_fp8(const void* x, const int32_t* pair_row, const int32_t* row_token,
                              const int32_t* nrows, int T, int H, int k, void* xg, float* scales,
                              float* stage, hipStream_t s);
+// Index pass and gather in one launch, for few pairs and rows that are not tiny
+// (small_permute_use); the same outputs, no workspace.
+bool small_permute_use(int T, int H, int k, int elem_bytes, bool fp8);
+hipError_t launch_small_permute(const void* x, int elem_bytes, bool fp8, const int32_t* ids, int T,
+                                int H, int E, int k, void* xg, float* scales, int32_t* row_token,
+                                int32_t* pair_row, int32_t* offsets, int32_t* counts,
+                                hipStream_t s);
 hipError_t launch_combine(const void* y, int y_dtype, const int32_t* pair_row, const float* w,
                           const void* shared, int T, int H, int k, void* out, hipStream_t s);
 

@@ -14,6 +14,7 @@
 // group with xor shuffles, and writes e4m3fn(clamp(x / s, +-448)) with
 // s = max(amax, 1e-10) / 448 into all k rows (16 bytes per lane), plus the
 // scale.
+#include "block_scan.h"
 #include "moe_common.h"
 #include <type_traits>
 
@@ -208,6 +209,145 @@ hipError_t launch_gather_fp8(const void* x, const int32_t* pair_row, const int32
   else
     hipLaunchKernelGGL(scatter_scales_kernel<1>, sgrid, dim3(256), 0, s, stage, row_token, nrows,
                        nitems, nb, T, scales);
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Small batches: the index pass and the gather in one launch.
+//
+// A decode batch's permute is a few thousand bytes of ids and a few rows; its
+// time is the launches (histogram, index, gather, fp8 scale copy: about 3 us
+// each on the host, as much on the device).  Here every block finds the rows of its own
+// pairs from all the ids: pair p of expert e goes to row
+//   #{q : (id_q, q) < (e, p)},
+// the stable expert-major order itself.  A thread holds up to kSmallPairs / 256
+// ids as keys id * kSmallPairs + q, so one pair costs one compare, ballot
+// and popcount per 64 ids.  One more block writes offsets and counts.
+// At most kSmallPairs pairs (half for the shortest rows, whose blocks rank the
+// pairs of five tokens) and rows of at least kSmallRowItems work items.
+// Measured (MI355X, us a call replayed from a graph, histogram + index + gather
+// launches / this one): bf16, E = 256, H = 7168, k = 8: T = 16 8.1 / 5.8, T = 256
+// 13.1 / 8.9; E = 8, H = 4096, k = 2: T = 64 7.5 / 3.2, T = 1024 9.9 / 6.6; fp8,
+// E = 256, H = 7168, k = 8, T = 128 15.4 / 6.9.  At 2048 pairs and H = 512 the
+// launch would tie the index and gather launches after a histogram handoff.
+// ---------------------------------------------------------------------------
+constexpr int kSmallPairs = 2048, kSmallRowItems = 64;
+constexpr int kSmallTok = 256 / kSmallRowItems + 1;  // tokens a block's items touch, at most
+
+template <int K, bool FP8>
+__global__ __launch_bounds__(256) void small_permute_kernel(
+    const u32x4* __restrict__ x, const int* __restrict__ ids, int npairs, int E, int k_rt,
+    int total, int per_row, u32x4* __restrict__ xg, float* __restrict__ scales,
+    int* __restrict__ row_token, int* __restrict__ pair_row, int* __restrict__ offsets,
+    int* __restrict__ counts) {
+  const int k = K > 0 ? K : k_rt;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nb = (int)gridDim.x - (offsets || counts ? 1 : 0);  // gather blocks
+  constexpr int IPT = kSmallPairs / 256;
+  int key[IPT];  // ids in (expert, pair) order; invalid ids and places past the end last
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) {
+    const int q = j * 256 + tid;
+    const int e = q < npairs ? ids[q] : -1;
+    key[j] = e >= 0 && e < E ? e * kSmallPairs + q : 0x7fffffff;
+  }
+  const int b = (int)blockIdx.x - ((int)gridDim.x - nb);
+  if (b < 0) {  // block 0: offsets and counts (the longest chain, so it goes first)
+    __shared__ int cnt[1024], offs[1025], sh4[4];
+    for (int e = tid; e < E; e += 256) cnt[e] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < IPT; ++j)
+      if (key[j] != 0x7fffffff) atomicAdd(&cnt[key[j] / kSmallPairs], 1);
+    __syncthreads();
+    lds_offsets(cnt, E, offs, sh4);
+    __syncthreads();
+    for (int e = tid; e <= E; e += 256) {
+      if (offsets) offsets[e] = offs[e];
+      if (counts && e < E) counts[e] = cnt[e];
+    }
+    return;
+  }
+  const int i0 = b * 256, i1 = min(i0 + 256, total);
+  const int t0 = i0 / per_row, t1 = (i1 - 1) / per_row;
+  const int np = (t1 - t0 + 1) * k;
+  __shared__ int part[4][kSmallTok * 8];
+  for (int p = 0; p < np; ++p) {
+    const int pair = t0 * k + p;
+    const int e = __builtin_amdgcn_readfirstlane(ids[pair]);
+    const int mine = (e >= 0 && e < E ? e : 0) * kSmallPairs + pair;
+    int c = 0;
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) c += __popcll(__ballot(key[j] < mine));
+    if (lane == 0) part[wave][p] = e >= 0 && e < E ? c : -npairs;  // stays negative when added
+  }
+  const int i = i0 + tid;
+  u32x4 val;
+  float scale = 0.0f;
+  const bool act = i < total;
+  if (act) {  // fp8: the 8 lanes of a block share a token (per_row % 8 == 0)
+    if constexpr (FP8) quant_chunk(x, i, val, scale);
+    else val = x[i];
+  }
+  __syncthreads();
+  if (!act) return;
+  const int t = i / per_row, v = i - t * per_row;
+  int r[K > 0 ? K : 8];
+#pragma unroll
+  for (int j = 0; j < (K > 0 ? K : 8); ++j) {
+    const int p = (t - t0) * k + j;
+    r[j] = K > 0 || j < k ? part[0][p] + part[1][p] + part[2][p] + part[3][p] : -1;
+    if (r[j] < 0) r[j] = -1;
+  }
+#pragma unroll
+  for (int j = 0; j < (K > 0 ? K : 8); ++j)
+    if (r[j] >= 0) st_nt(xg + (long long)r[j] * per_row + v, val);
+  if constexpr (FP8) {
+    if ((v & 7) == 0) {
+#pragma unroll
+      for (int j = 0; j < (K > 0 ? K : 8); ++j)
+        if (r[j] >= 0) scales[(long long)r[j] * (per_row / 8) + v / 8] = scale;
+    }
+  }
+  if (v == 0) {
+#pragma unroll
+    for (int j = 0; j < (K > 0 ? K : 8); ++j) {
+      if (K == 0 && j >= k) break;
+      pair_row[t * k + j] = r[j];
+      if (r[j] >= 0) row_token[r[j]] = t;
+    }
+  }
+}
+
+bool small_permute_use(int T, int H, int k, int elem_bytes, bool fp8) {
+  const int per_row = fp8 ? H / 16 : (int)((long long)H * elem_bytes / 16);
+  return T > 0 && per_row >= kSmallRowItems &&
+         (long long)T * k <= (per_row >= 2 * kSmallRowItems ? kSmallPairs : kSmallPairs / 2);
+}
+
+hipError_t launch_small_permute(const void* x, int elem_bytes, bool fp8, const int32_t* ids, int T,
+                                int H, int E, int k, void* xg, float* scales, int32_t* row_token,
+                                int32_t* pair_row, int32_t* offsets, int32_t* counts,
+                                hipStream_t s) {
+  const int per_row = fp8 ? H / 16 : (int)((long long)H * elem_bytes / 16);
+  const int total = T * per_row;  // < 2^31, checked by the caller
+  const dim3 grid((unsigned)((total + 255) / 256 + (offsets || counts ? 1 : 0))), blk(256);
+#define MOE_SMALL(KK)                                                                         \
+  {                                                                                           \
+    if (fp8)                                                                                  \
+      hipLaunchKernelGGL((small_permute_kernel<KK, true>), grid, blk, 0, s, (const u32x4*)x, ids, \
+                         T * k, E, k, total, per_row, (u32x4*)xg, scales, row_token, pair_row, \
+                         offsets, counts);                                                    \
+    else                                                                                      \
+      hipLaunchKernelGGL((small_permute_kernel<KK, false>), grid, blk, 0, s, (const u32x4*)x, ids, \
+                         T * k, E, k, total, per_row, (u32x4*)xg, scales, row_token, pair_row, \
+                         offsets, counts);                                                    \
+  }
+  if (k == 8) MOE_SMALL(8)
+  else if (k == 2) MOE_SMALL(2)
+  else MOE_SMALL(0)
+#undef MOE_SMALL
   return hipGetLastError();
 }
 
