@@ -22,7 +22,7 @@
 // group_counts[r / group_rows] == 0 (the weights of experts that received no
 // rows are never read).
 //
-// Layout: 256-thread blocks (at most 8 per CU), which walk the rows of the
+// Layout: 256-thread blocks, which walk the rows of the
 // non-empty groups only (listed per block in LDS), RB consecutive rows per pass
 // (RB = 4 / 2 / 1 for K up to 4096 / 8192 / 16384) and issuing all their
 // loads before the first reduction; for one row, thread t holds 16 consecutive
@@ -36,7 +36,14 @@ namespace moe {
 
 constexpr int kQuantThreads = 256;
 constexpr int kQuantChunk = kQuantThreads * 16;  // elements per chunk
-constexpr int kQuantBlocks = 256 * 8;            // 8 resident blocks per CU
+// Blocks at most.  A block that loops waits for its stores' rows before the next
+// rows' loads, so many short blocks overlap better than 8 resident ones per CU;
+// a block per pass costs more where most groups are empty.  Gate weights of 64
+// experts (3584 x 8192 each, us; all groups / 8 of them), 8 / 32 / 64 / 128 blocks
+// per CU and one per pass: 1039 / 1020 / 995 / 981 / 948, and 118 / 112 / 114 /
+// 119 / 145.  With plain stores instead of st_sc1 (the int8 rows are read again by
+// the GEMM, 1.9 GB later) 1073 at 8.
+constexpr int kQuantBlocks = 256 * 128;
 constexpr int kQuantMaxGroups = 4096;            // groups gated by group_counts
 
 // v of lane (lane ^ m), m in {1, 2, 4}, through DPP moves (no LDS traffic):
@@ -170,7 +177,7 @@ __global__ __launch_bounds__(kQuantThreads) void quant_rows_i8_kernel(
           }
           out[w] = pk;
         }
-        *reinterpret_cast<u32x4*>(qr + e0) = out;
+        st_sc1(reinterpret_cast<u32x4*>(qr + e0), out);
       }
     }
     __syncthreads();  // part[] is rewritten by the next pass
