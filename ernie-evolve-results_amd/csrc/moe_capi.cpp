@@ -234,7 +234,7 @@ static int route_launch(const void* x, const void* w, int w_dtype, const float* 
                     "topk");
   }
   const int N = w_dtype == MOE_DTYPE_FP32 ? 2 * E : E;
-  const int ksplit = moe::router_gemm_ksplit(T, H, N);
+  const int ksplit = moe::router_gemm_ksplit_run(T, H, N);
   const int parts = (N / E) * ksplit;
   const __bf16* wb = (const __bf16*)w;
   char* wsp = (char*)ws;

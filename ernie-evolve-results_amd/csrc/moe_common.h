@@ -51,7 +51,9 @@ namespace moe {
 hipError_t launch_wsplit(const float* w, __bf16* wpk, int E, int H, hipStream_t s);
 hipError_t launch_router_gemm(const __bf16* x, const __bf16* w, int T, int H, int N,
                               int ksplit, float* out, hipStream_t s);
+// K partitions: the most a launch uses (sizes the workspace), and those it does.
 int router_gemm_ksplit(int T, int H, int N);
+int router_gemm_ksplit_run(int T, int H, int N);
 // The router GEMM with K split over the waves of a block (router_wk.hip), for
 // batches too small to fill the chip with whole-K tiles: whether (T, H, E) takes
 // it, and its launch (w bf16 [E, H], or with wf32 fp32 [E, H] split hi/lo in the

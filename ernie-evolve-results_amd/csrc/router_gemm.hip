@@ -67,7 +67,7 @@ hipError_t launch_wsplit(const float* w, __bf16* wpk, int E, int H, hipStream_t 
 template <int BM, int BN, int NS, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN) void router_gemm_dma_kernel(
     const __bf16* __restrict__ x, const __bf16* __restrict__ w, int T, int H, int N,
-    int kchunk, float* __restrict__ out, int ldo) {
+    float* __restrict__ out, int ldo) {
   constexpr int BK = 64, CH = 8, ROWB = 128, RPI = 8;
   constexpr int STAGE_B = (BM + BN) * ROWB;
   constexpr int A_INST = BM / RPI, B_INST = BN / RPI, NW = WM * WN;
@@ -82,8 +82,10 @@ __global__ __launch_bounds__(64 * WM * WN) void router_gemm_dma_kernel(
   const int wm = wave / WN, wn = wave % WN;
   const long long m0 = (long long)blockIdx.x * BM;
   const int n0 = blockIdx.y * BN;
-  const int kb = blockIdx.z * kchunk;
-  const int KT = kchunk / BK;
+  // K partition z of gridDim.z: whole 64-wide steps, as even as they go
+  const int U = H / BK, z = blockIdx.z, nz = gridDim.z;
+  const int kb = (int)((long long)z * U / nz) * BK;
+  const int KT = (int)((long long)(z + 1) * U / nz) - kb / BK;
   auto swz = [](int r) { return (r >> 1) & (CH - 1); };
 
   // Per-lane source of each of this wave's DMA instructions (row clamped
@@ -176,7 +178,7 @@ static hipError_t launch_dma(const __bf16* x, const __bf16* w, int T, int H, int
                              float* out, hipStream_t s) {
   const dim3 grid((unsigned)((T + BM - 1) / BM), (unsigned)((N + BN - 1) / BN), (unsigned)ksplit);
   hipLaunchKernelGGL((router_gemm_dma_kernel<BM, BN, NS, WM, WN>), grid, dim3(64 * WM * WN), 0,
-                     s, x, w, T, H, N, H / ksplit, out, N * ksplit);
+                     s, x, w, T, H, N, out, N * ksplit);
   return hipGetLastError();
 }
 
@@ -201,8 +203,32 @@ int router_gemm_ksplit(int T, int H, int N) {
   return ks;
 }
 
+// The partitions a launch uses, at most router_gemm_ksplit (which sizes the
+// workspace): the count whose rounds of 256 blocks are shortest.  A doubling that
+// just passes the target leaves a second, nearly empty round: E = 64 with fp32
+// weights (N = 128), H = 8192, T = 4904 has 77 row tiles, so 4 partitions are 308
+// blocks and 3 are 231; T = 4133 260 and 195 (route 46.3 / 37.5 us).  E = 256,
+// H = 8192: T = 4133 60.7 / 49.0, 6000 68.0 / 52.7; E = 256, H = 4096, fp32 weights:
+// T = 4133 64.7 / 50.9.
+int router_gemm_ksplit_run(int T, int H, int N) {
+  const GemmTile g = gemm_tile(N);
+  const long long blocks = (long long)((T + g.bm - 1) / g.bm) * ((N + g.bn - 1) / g.bn);
+  const int most = router_gemm_ksplit(T, H, N);
+  if (N < 128) return most;  // three or more of these blocks share a CU: no rounds
+  int best = 1;
+  long long br = (blocks + 255) / 256;
+  for (int ks = 2; ks <= most; ++ks) {
+    const long long r = (blocks * ks + 255) / 256;
+    if (r * best <= br * ks) {  // rounds / partitions: no longer
+      best = ks;
+      br = r;
+    }
+  }
+  return best;
+}
+
 // N in {8, 16, 32, 64, 128} or a multiple of 256; H % 64 == 0 (checked by
-// the caller); H % (64 * ksplit) == 0.
+// the caller); ksplit at most H / 64.
 hipError_t launch_router_gemm(const __bf16* x, const __bf16* w, int T, int H, int N, int ksplit,
                               float* out, hipStream_t s) {
   if (N >= 256) return launch_dma<256, 128, 3, 4, 4>(x, w, T, H, N, ksplit, out, s);

@@ -110,3 +110,17 @@ def test_fused_kernel_block_histograms(cuda, E, H, T, k):
     p = M.permute(x, plan.topk_ids, E, index_only=True)
     for name in ("row_token", "pair_row", "offsets", "counts"):
         assert torch.equal(getattr(plan, name), p[name]), name
+
+
+@pytest.mark.parametrize("E,H,T,fp32", [(64, 8192, 4133, True), (64, 8192, 4904, True),
+                                        (256, 8192, 4133, False), (256, 8256, 5000, False),
+                                        (128, 4160, 6001, True), (256, 1088, 1100, True)])
+def test_uneven_k_partitions(cuda, E, H, T, fp32):
+    """K split over blocks into 3 to 7 parts of unequal length, the partial sums
+    added by the scoring kernel."""
+    x, w = inputs(T, H, E, T + E, cuda)
+    w = w if fp32 else w.bfloat16()
+    logits, ids, wts, counts = M.route(x, w, None, 8, RouteCfg())
+    assert_logits(logits, x, w, fp32)
+    i2, w2, c2 = M.topk(logits, None, 8, RouteCfg())
+    assert torch.equal(ids, i2) and torch.equal(wts, w2) and torch.equal(counts, c2)
