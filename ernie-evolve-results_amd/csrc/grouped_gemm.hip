@@ -37,12 +37,19 @@
 // bf16 1292 / 1489, SwiGLU 1337 / 1501, int8 2623 / 2854; 65536 x 8192 x 3584 bf16
 // 1310 / 1451, int8 2268 / 2455.  The rest is the clock: 1.48 GHz at this load.
 // The routed experts (64 experts, H = 8192, Ni = 3584, top-8, us): gate+up T = 16
-// 1229 / 1136, 1024 1794 / 1313, 2048 2398 / 2073; the 128 x 512 tiles that small
-// groups had are slower everywhere but the int8 down projection at T = 16 ..
-// 768 (332 / 356 at T = 64).  Tried and slower: four half steps of 16 MFMAs (5%
-// instead of 13% gained), s_setprio around the MFMAs (-1%), the DMA issued
+// 1229 / 1122, 1024 1794 / 1340, 2048 2398 / 2070; the 128 x 512 tiles that small
+// groups had are slower everywhere.  Tried and slower: four half steps of 16 MFMAs
+// (5% instead of 13% gained), s_setprio around the MFMAs (-1%), the DMA issued
 // between the MFMAs (-8%), the closing barrier 2 .. 12 MFMAs early (-8 .. -12%),
 // 32x32x16 MFMAs (-13%).
+//
+// Tiles of at most 128 rows, where groups are small on average (bf16 and int8), are
+// bound by their weight loads: all waves step together through a ring of three
+// stages of 48 KB (128 rows) or four of 40 KB (64 rows), one barrier a step, so 64 or
+// 96 KB of weights are in flight instead of 48.  Against the loop above: down
+// T = 16 592 / 573, 64 630 / 619; int8 gate+up T = 16 659 / 624, down T = 64 353 /
+// 338; nothing at 1024 rows per group.  Row tiles of equal height instead of a last
+// one with the rest: no gain (2041 / 2018 .. 2027 at T = 2048).
 //
 // fp8 A: the DMA brings each wave's own 16 rows of e4m3fn bytes, and half a K step
 // before they are read the wave writes them once as bf16(q * s) into the A tile
@@ -305,7 +312,11 @@ template <GgType TY> __device__ constexpr int a_at(int buf, int x) {
 }
 __device__ constexpr int raw_at(int buf, int x) { return 6 * kHalf + (buf * 2 + x) * kRaw; }
 __device__ constexpr int sc_at(int buf, int x) { return 8 * kHalf + (buf * 2 + x) * 2048; }
-template <GgType TY> constexpr int kLds = TY == kFp8 ? 8 * kHalf + 8192 : 8 * kHalf;
+// bf16 / int8 tiles of at most 128 rows: stages of B0, B1 and 128 or 64 rows of A
+constexpr int kShort128 = 3 * kHalf, kShort64 = 2 * kHalf + kHalf / 2;
+template <GgType TY, bool SHORT>
+constexpr int kLds = TY == kFp8 ? 8 * kHalf + 8192 : SHORT ? 4 * kShort64 : 8 * kHalf;
+static_assert(4 * kShort64 >= 8 * kHalf && 4 * kShort64 >= 3 * kShort128, "LDS map");
 
 template <int N>
 __device__ __forceinline__ void wait_vm() {
@@ -326,7 +337,8 @@ __device__ __forceinline__ void dma4(const char* src, char* dst) {
 }
 }  // namespace gg
 
-template <bool SWIGLU, GgType TY>
+// SHORT: tiles of at most 128 rows take the ring loop.
+template <bool SWIGLU, GgType TY, bool SHORT>
 __global__ __launch_bounds__(512) void grouped_gemm_kernel(
     const char* __restrict__ a, const char* __restrict__ ident_a, int ident_m,
     const char* __restrict__ w0, const char* __restrict__ w1, const int* __restrict__ offs,
@@ -336,7 +348,7 @@ __global__ __launch_bounds__(512) void grouped_gemm_kernel(
   constexpr bool I8 = TY == kInt8, F8 = TY == kFp8;
   constexpr int EL = I8 ? 1 : 2;       // bytes per weight element
   constexpr int BM = kGgBM;
-  __shared__ __attribute__((aligned(1024))) char lds[kLds<TY>];
+  __shared__ __attribute__((aligned(1024))) char lds[kLds<TY, SHORT>];
   GgTile tile;
   if (!gg_tile<BM>(offs, tile_start, G, M, n_tiles, ident_m, tile)) return;
   // wave-uniform: in SGPRs
@@ -480,93 +492,167 @@ __global__ __launch_bounds__(512) void grouped_gemm_kernel(
   };
 
   const int KT = K * EL / 128;
-  issue_b(0, 0);
-  issue_a(0, 0);
-  if constexpr (F8) issue_s(0, 0);
-  issue_b(1, 0);
-  issue_a(1, 0);
-  if constexpr (F8) issue_s(1, 0);
-  if (KT > 1) {
-    issue_b(0, 1);
-    issue_a(0, 1);
-    issue_b(1, 1);
-    if constexpr (F8) {
-      issue_a(1, 1);
-      wait_vm<6>();  // step 0 landed
-    } else {
-      wait_vm<8>();  // B0, A0 and B1 of step 0 landed
-    }
-  } else {
-    wait_vm<2>();  // not fp8 (K % 128 == 0): all but A1
-  }
-  barrier();
-  read_b(fb0[0], 0, 0);
-  if constexpr (F8) convert(0, 0, 0);
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  barrier();
-  if (wm == 1) barrier();  // half a step behind the other group from here on
-  // P: parity of the step; rem: steps after it; sb (fp8): scale buffer of the step
-  auto step = [&]<int P>(std::integral_constant<int, P>, int rem, int sb)
-                  __attribute__((always_inline)) {
-    read_a(0, P);
-    read_b(fb1, 1, P);
-    if constexpr (F8) {
-      convert(1, P, sb);
-      // per half step B0 + raw A0 or B1 + raw A1 (3 loads), in even steps a scale
-      // too: what the next half needs was issued two half steps ago
-      if (rem >= 2) {
-        issue_b(0, P);
-        issue_a(0, P);
-        if (P == 0) issue_s(0, sb ^ 1);
-        wait_vm<7>();
-      } else if (P == 0) {
-        wait_vm<3>();
-      } else {
-        wait_vm<0>();
+  const int rows = rlast + 1 - r0;  // of this tile, 256 if more
+  // A tile of at most RA = 128 or 64 rows (a small group, or a group's last tile):
+  // the loads bound it, so all waves step together through a ring of NB stages of
+  // RA rows of A and the 256 weight rows, one barrier a step, NB - 1 steps in
+  // flight.  The same wave -> row and column map, so the waves of rows past RA
+  // (and the second row half) have nothing to multiply.
+  auto short_loop = [&]<int RA, int NB>(std::integral_constant<int, RA>,
+                                        std::integral_constant<int, NB>)
+                        __attribute__((always_inline)) {
+    constexpr int STAGE = 2 * kHalf + RA * 128;
+    const bool loads_a = wave * 16 < RA;
+    auto issue = [&](int st) __attribute__((always_inline)) {
+      char* d = lds + st * STAGE + wave * 2048;
+#pragma unroll
+      for (int y = 0; y < 2; ++y)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          dma16(bsrc[y][q], d + y * kHalf + q * 1024);
+          bsrc[y][q] += 128;
+        }
+      if (loads_a) {
+#pragma unroll
+        for (int q = 0; q < NA; ++q) {
+          dma16(asrc[0][q], d + 2 * kHalf + q * 1024);
+          asrc[0][q] += 128;
+        }
       }
-    } else {
-      // in flight after the loads that the next half needs (A1 of this step, B0 of
-      // the next): A0 and B1 of the next step and the two elements issued here
-      if (rem >= 2) {
-        issue_a(1, P ^ 1);
-        issue_b(0, P);
-        wait_vm<8>();
-      } else if (rem == 1) {
-        issue_a(1, P ^ 1);
-        wait_vm<6>();
-      } else {
-        wait_vm<0>();
+    };
+    int st_in = 0, st = 0;
+    for (; st_in < NB - 1 && st_in < KT; ++st_in) issue(st_in);
+    st_in = NB - 1;
+    for (int kt = 0; kt < KT; ++kt) {
+      // this wave's part of the step landed once at most NB - 2 later ones are
+      // outstanding; the barrier makes that true for every wave, and every wave is
+      // past its reads of the stage refilled now
+      if (kt + NB - 2 >= KT) wait_vm<0>();
+      else if (loads_a) wait_vm<(NB - 2) * 6>();
+      else wait_vm<(NB - 2) * 4>();
+      barrier();
+      if (kt + NB - 1 < KT) issue(st_in);
+      if (live0) {
+        const char* p = lds + st * STAGE;
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            fa[kk][i] = *reinterpret_cast<const bf16x8*>(p + 2 * kHalf + aoff[kk] + i * 2048);
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            fb0[0][kk][j] = *reinterpret_cast<const bf16x8*>(p + boff[kk] + j * 2048);
+            fb1[kk][j] = *reinterpret_cast<const bf16x8*>(p + kHalf + boff[kk] + j * 2048);
+          }
+        }
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+          for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+              for (int j = 0; j < 2; ++j)
+                acc[0][y][i][j] =
+                    mfma_step<I8>(fa[kk][i], y ? fb1[kk][j] : fb0[0][kk][j], acc[0][y][i][j]);
       }
+      st = st == NB - 1 ? 0 : st + 1;
+      st_in = st_in == NB - 1 ? 0 : st_in + 1;
     }
-    mma(0, fb0[P], live0);
-    read_a(1, P);
-    read_b(fb0[P ^ 1], 0, P ^ 1);  // past the last step: not used
-    if constexpr (F8) {
-      if (rem >= 1) convert(0, P ^ 1, P == 0 ? sb : sb ^ 1);
-      if (rem >= 2) {
-        issue_b(1, P);
-        issue_a(1, P);
-        if (P == 0) issue_s(1, sb ^ 1);
-        wait_vm<P == 0 ? 8 : 6>();
-      } else {
-        wait_vm<0>();
-      }
-    } else if (rem >= 2) {
-      issue_a(0, P);
-      issue_b(1, P);
-      wait_vm<8>();
-    } else {
-      wait_vm<2>();  // rem 1: A1 of the last step may still be in flight
-    }
-    mma(1, fb0[P], live1);
   };
-  int sb = 0;
-  for (int kt = 0; kt < KT; kt += 2) {
-    step(std::integral_constant<int, 0>{}, KT - 1 - kt, sb);
-    if (F8 || kt + 1 < KT) step(std::integral_constant<int, 1>{}, KT - 2 - kt, sb);
-    if (F8) sb ^= 1;
+  if (SHORT && rows <= 64) {
+    if constexpr (SHORT) short_loop(std::integral_constant<int, 64>{}, std::integral_constant<int, 4>{});
+  } else if (SHORT && rows <= 128) {
+    if constexpr (SHORT) short_loop(std::integral_constant<int, 128>{}, std::integral_constant<int, 3>{});
+  } else {
+    issue_b(0, 0);
+    issue_a(0, 0);
+    if constexpr (F8) issue_s(0, 0);
+    issue_b(1, 0);
+    issue_a(1, 0);
+    if constexpr (F8) issue_s(1, 0);
+    if (KT > 1) {
+      issue_b(0, 1);
+      issue_a(0, 1);
+      issue_b(1, 1);
+      if constexpr (F8) {
+        issue_a(1, 1);
+        wait_vm<6>();  // step 0 landed
+      } else {
+        wait_vm<8>();  // B0, A0 and B1 of step 0 landed
+      }
+    } else {
+      wait_vm<2>();  // not fp8 (K % 128 == 0): all but A1
+    }
+    barrier();
+    read_b(fb0[0], 0, 0);
+    if constexpr (F8) convert(0, 0, 0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    barrier();
+    if (wm == 1) barrier();  // half a step behind the other group from here on
+    // P: parity of the step; rem: steps after it; sb (fp8): scale buffer of the step
+    auto step = [&]<int P>(std::integral_constant<int, P>, int rem, int sb)
+                    __attribute__((always_inline)) {
+      read_a(0, P);
+      read_b(fb1, 1, P);
+      if constexpr (F8) {
+        convert(1, P, sb);
+        // per half step B0 + raw A0 or B1 + raw A1 (3 loads), in even steps a scale
+        // too: what the next half needs was issued two half steps ago
+        if (rem >= 2) {
+          issue_b(0, P);
+          issue_a(0, P);
+          if (P == 0) issue_s(0, sb ^ 1);
+          wait_vm<7>();
+        } else if (P == 0) {
+          wait_vm<3>();
+        } else {
+          wait_vm<0>();
+        }
+      } else {
+        // in flight after the loads that the next half needs (A1 of this step, B0 of
+        // the next): A0 and B1 of the next step and the two elements issued here
+        if (rem >= 2) {
+          issue_a(1, P ^ 1);
+          issue_b(0, P);
+          wait_vm<8>();
+        } else if (rem == 1) {
+          issue_a(1, P ^ 1);
+          wait_vm<6>();
+        } else {
+          wait_vm<0>();
+        }
+      }
+      mma(0, fb0[P], live0);
+      read_a(1, P);
+      read_b(fb0[P ^ 1], 0, P ^ 1);  // past the last step: not used
+      if constexpr (F8) {
+        if (rem >= 1) convert(0, P ^ 1, P == 0 ? sb : sb ^ 1);
+        if (rem >= 2) {
+          issue_b(1, P);
+          issue_a(1, P);
+          if (P == 0) issue_s(1, sb ^ 1);
+          wait_vm<P == 0 ? 8 : 6>();
+        } else {
+          wait_vm<0>();
+        }
+      } else if (rem >= 2) {
+        issue_a(0, P);
+        issue_b(1, P);
+        wait_vm<8>();
+      } else {
+        wait_vm<2>();  // rem 1: A1 of the last step may still be in flight
+      }
+      mma(1, fb0[P], live1);
+    };
+    int sb = 0;
+    for (int kt = 0; kt < KT; kt += 2) {
+      step(std::integral_constant<int, 0>{}, KT - 1 - kt, sb);
+      if (F8 || kt + 1 < KT) step(std::integral_constant<int, 1>{}, KT - 2 - kt, sb);
+      if (F8) sb ^= 1;
+    }
+    if (wm == 0) barrier();
   }
-  if (wm == 0) barrier();
 
   // ---- epilogue: element e of a 16 x 16 block is row fc*4 + e, column fr.
   // SwiGLU: B half 0 is the gate, half 1 the up product of the same columns.
@@ -673,14 +759,25 @@ static hipError_t launch_gg(const void* a, const void* ident_a, int ident_m, con
   const int n_tiles = grouped_gemm_n_tiles(N, swiglu);
   const long long blocks = (((long long)M + kGgBM - 1) / kGgBM + G) * n_tiles;
   const dim3 grid((unsigned)((blocks + 7) / 8 * 8)), blk(512);
-  if (swiglu)
-    hipLaunchKernelGGL((grouped_gemm_kernel<true, TY>), grid, blk, 0, s, (const char*)a,
-                       (const char*)ident_a, ident_m, (const char*)w0, (const char*)w1, offs,
-                       tile_start, G, M, N, K, n_tiles, (unsigned short*)out, ex);
-  else
-    hipLaunchKernelGGL((grouped_gemm_kernel<false, TY>), grid, blk, 0, s, (const char*)a,
-                       (const char*)ident_a, ident_m, (const char*)w0, (const char*)w0, offs,
-                       tile_start, G, M, N, K, n_tiles, (unsigned short*)out, ex);
+  // Groups of at most 128 rows on average: the kernel with the ring loop for short
+  // tiles.  The one without it keeps 0.3 .. 0.6% at T = 8192 (whole layer 10.31 /
+  // 10.36 ms; it needs 256 registers and 160 KB of LDS), the one with it gains 2.8%
+  // at T = 16 (1671 / 1625 us).
+  constexpr bool kRing = TY != kFp8;
+  const bool ring = kRing && (long long)M <= 128ll * G;
+#define MOE_GG(SW, SH)                                                                         \
+  hipLaunchKernelGGL((grouped_gemm_kernel<SW, TY, SH>), grid, blk, 0, s, (const char*)a,        \
+                     (const char*)ident_a, ident_m, (const char*)w0,                           \
+                     (const char*)(swiglu ? w1 : w0), offs, tile_start, G, M, N, K, n_tiles,   \
+                     (unsigned short*)out, ex)
+  if (swiglu) {
+    if (ring) MOE_GG(true, kRing);
+    else MOE_GG(true, false);
+  } else {
+    if (ring) MOE_GG(false, kRing);
+    else MOE_GG(false, false);
+  }
+#undef MOE_GG
   return hipGetLastError();
 }
 

@@ -13,7 +13,10 @@ import moe_route as M
 
 pytestmark = pytest.mark.gpu
 
-ENDS = [1, 64, 129, 129, 320, 577, 833, 1100]  # 1, 63, 65, 0, 191, 257, 256, 267 rows
+BASE = [1, 64, 129, 129, 320, 577, 833, 1100]  # 1, 63, 65, 0, 191, 257, 256, 267 rows
+# 137 rows a group on average; with empty groups added, few enough that short tiles
+# (64 and 128 rows) take the ring loop
+EMPTY = [0, 8]
 
 
 def groups(ends, rows):
@@ -23,18 +26,20 @@ def groups(ends, rows):
         lo = hi
 
 
-def make(K, N, dev, seed):
+def make(K, N, dev, seed, empty):
+    ENDS = BASE + BASE[-1:] * empty
     g = torch.Generator(device=dev).manual_seed(seed)
     rows = ENDS[-1] + 30  # the last rows belong to no group
     a = torch.randn(rows, K, generator=g, device=dev).bfloat16()
     w = torch.randn(len(ENDS), N, K, generator=g, device=dev).bfloat16()
-    return a, w, torch.tensor(ENDS, dtype=torch.int32, device=dev)
+    return a, w, torch.tensor(ENDS, dtype=torch.int32, device=dev), ENDS
 
 
+@pytest.mark.parametrize("empty", EMPTY)
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 320])
 @pytest.mark.parametrize("N", [256, 264, 131])
-def test_bf16(cuda, K, N):
-    a, w, offs = make(K, N, cuda, K + N)
+def test_bf16(cuda, K, N, empty):
+    a, w, offs, ENDS = make(K, N, cuda, K + N, empty)
     out = torch.full((a.shape[0], N), 7.0, dtype=torch.bfloat16, device=cuda)
     M.grouped_gemm(a, w, offs, out=out)
     for g, lo, hi in groups(ENDS, a.shape[0]):
@@ -45,10 +50,11 @@ def test_bf16(cuda, K, N):
     assert bool((out[ENDS[-1]:] == 7.0).all())
 
 
+@pytest.mark.parametrize("empty", EMPTY)
 @pytest.mark.parametrize("K", [128, 256, 384, 512])
 @pytest.mark.parametrize("N", [256, 131])
-def test_int8(cuda, K, N):
-    a, w, offs = make(K, N, cuda, K * 3 + N)
+def test_int8(cuda, K, N, empty):
+    a, w, offs, ENDS = make(K, N, cuda, K * 3 + N, empty)
     q, s = M.quant_rows_i8(a)
     wq, ws = M.quant_rows_i8(w)
     out = torch.full((a.shape[0], N), 7.0, dtype=torch.bfloat16, device=cuda)
@@ -60,11 +66,12 @@ def test_int8(cuda, K, N):
     assert bool((out[ENDS[-1]:] == 7.0).all())
 
 
+@pytest.mark.parametrize("empty", EMPTY)
 @pytest.mark.parametrize("K", [128, 256, 384])
 @pytest.mark.parametrize("N", [256, 131])
 @pytest.mark.parametrize("swiglu", [False, True])
-def test_fp8_matches_bf16_on_dequantised_rows(cuda, K, N, swiglu):
-    a, w, offs = make(K, N, cuda, K * 5 + N)
+def test_fp8_matches_bf16_on_dequantised_rows(cuda, K, N, swiglu, empty):
+    a, w, offs, ENDS = make(K, N, cuda, K * 5 + N, empty)
     p = M.permute(a, torch.zeros(a.shape[0], 1, dtype=torch.int32, device=cuda), 1, fp8=True)
     q, s = p["xg"], p["scales"]
     deq = (q.view(torch.float8_e4m3fn).float().view(a.shape[0], -1, 128) * s[..., None]).view(
