@@ -37,19 +37,28 @@
 // bf16 1292 / 1489, SwiGLU 1337 / 1501, int8 2623 / 2854; 65536 x 8192 x 3584 bf16
 // 1310 / 1451, int8 2268 / 2455.  The rest is the clock: 1.48 GHz at this load.
 // The routed experts (64 experts, H = 8192, Ni = 3584, top-8, us): gate+up T = 16
-// 1229 / 1122, 1024 1794 / 1340, 2048 2398 / 2070; the 128 x 512 tiles that small
-// groups had are slower everywhere.  Tried and slower: four half steps of 16 MFMAs
-// (5% instead of 13% gained), s_setprio around the MFMAs (-1%), the DMA issued
+// 1229 / 1122, 1024 1794 / 1340, 2048 2398 / 2070.  Tried and slower: four half steps
+// of 16 MFMAs (5% instead of 13% gained), s_setprio around the MFMAs (-1%), the DMA issued
 // between the MFMAs (-8%), the closing barrier 2 .. 12 MFMAs early (-8 .. -12%),
 // 32x32x16 MFMAs (-13%).
 //
 // Tiles of at most 128 rows, where groups are small on average (bf16 and int8), are
-// bound by their weight loads: all waves step together through a ring of three
-// stages of 48 KB (128 rows) or four of 40 KB (64 rows), one barrier a step, so 64 or
-// 96 KB of weights are in flight instead of 48.  Against the loop above: down
-// T = 16 592 / 573, 64 630 / 619; int8 gate+up T = 16 659 / 624, down T = 64 353 /
-// 338; nothing at 1024 rows per group.  Row tiles of equal height instead of a last
-// one with the rest: no gain (2041 / 2018 .. 2027 at T = 2048).
+// bound by their weight loads, and with few K steps by the start and end of a block: a
+// CU holds one, so nothing else overlaps them.  All waves step together through a ring of
+// three stages of up to 48 KB, one barrier a step; only the 16-row blocks that exist are
+// computed and stored, from registers; a block can take two column tiles in a row
+// (grouped_runs.h); and its tile is found by DPP scans.  Measured (us; experts of N x K
+// weights, 128 x 512 tiles with a two-stage loop / 256-row tiles with the epilogue of 256
+// rows / this): int8 128 experts 2048 x 512, 4 rows each 38 / 55 / 28, 40 rows
+// 40 / 59 / 34; 64 experts SwiGLU 2048 x 1024, 16 rows 60 / 82 / 45; bf16 128 experts
+// 1024 x 512, 16 rows 29 / 34 / 26; 64 experts SwiGLU 1024 x 1024, 4 rows 48 / 52 / 43;
+// 8 experts SwiGLU 2048 x 4096, 16 rows 95 / 49 / 45.  Where the 128 x 512 tiles fill
+// whole rounds of CUs and the weights' rows are a power of two apart they stay 3 .. 6%
+// ahead: bf16 64 experts 4096 x 2048, 16 rows 188 / 206 / 196; SwiGLU 2048 x 4096, 40 rows
+// 363 / 382 / 378; 128 experts 1024 x 512, 100 rows 33 / 40 / 34.4.  Tried: four stages of
+// 40 KB at up to 64 rows (no gain), two steps loaded at a time (-4%), other orders of the
+// tiles over the XCDs (-2 .. -30%), row tiles of equal height instead of a last one with
+// the rest (no gain: 2041 / 2018 .. 2027 at T = 2048).
 //
 // fp8 A: the DMA brings each wave's own 16 rows of e4m3fn bytes, and half a K step
 // before they are read the wave writes them once as bf16(q * s) into the A tile
@@ -68,7 +77,9 @@
 // Identity shortcut (the reference's ident_a / ident_m): a group whose row
 // count equals ident_m takes its A rows from ident_a (row i of the group =
 // row i of ident_a) instead of a.
+#include "grouped_runs.h"
 #include "moe_common.h"
+#include <cmath>
 #include <utility>
 
 namespace moe {
@@ -126,24 +137,22 @@ __global__ __launch_bounds__(1024) void gg_plan_kernel(const int* __restrict__ o
 // output (a chain of dependent loads at the start of every tile).
 constexpr int kScanG = 256;
 
-// Row tiles of group gi (ends clamped into [0, M], as the tile itself does);
-// 0 past G.
-__device__ __forceinline__ int group_tiles(const int* __restrict__ offs, int gi, int G, int M,
-                                           int bm) {
-  if (gi >= G) return 0;
-  const int lo = gi > 0 ? min(max(offs[gi - 1], 0), M) : 0;
-  const int hi = min(max(offs[gi], 0), M);
-  return hi > lo ? (hi - lo + bm - 1) / bm : 0;
+// Rows [lo, hi) of group gi, its ends clamped into [0, M]; empty past G.
+__device__ __forceinline__ void group_rows(const int* __restrict__ offs, int gi, int G, int M,
+                                           int& lo, int& hi) {
+  lo = gi > 0 && gi < G ? min(max(offs[gi - 1], 0), M) : 0;
+  hi = gi < G ? max(min(max(offs[gi], 0), M), lo) : lo;
 }
 
-// Inclusive wave scan.
+// Inclusive wave scan by DPP moves (no LDS latency: it is on the way to a tile's first
+// load): in rows of 16 lanes, then the row sums across rows.
 __device__ __forceinline__ int wave_incl_scan(int v) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int n = __shfl_up(v, o, 64);
-    if (lane >= o) v += n;
-  }
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast15, 31
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
   return v;
 }
 
@@ -191,19 +200,23 @@ struct GgExtra {
   const float* w1;     // [G, N] per weight row of w1 (SwiGLU up)
 };
 
-// The tile of block blockIdx.x: false if the block has none.  BM rows per tile.
+// The tiles of block blockIdx.x: false if it has none.  BM rows per tile.
 struct GgTile {
   int g;      // group
   int gs;     // its first row
   int r0;     // first row of the tile
   int rlast;  // last row of the group
-  int nt;     // column tile
+  int nt, nt1; // column tiles [nt, nt1)
+  int rot;     // which of them comes first
   bool ident; // A rows from ident_a
 };
-template <int BM>
+// RUN: gg_run column tiles per block in short groups, by the real tile counts (up to
+// kScanG groups, fewer than 2^15 row tiles; beyond, one).
+template <int BM, bool RUN>
 __device__ __forceinline__ bool gg_tile(const int* __restrict__ offs,
                                         const int* __restrict__ tile_start, int G, int M,
-                                        int n_tiles, int ident_m, GgTile& out) {
+                                        int n_tiles, int KT, int ident_m,
+                                        GgTile& out) {
   // XCD-aware order: hardware block b runs on XCD b % 8.  The grid is sized
   // by a bound on the tile count; the real count nreal is known here, and the
   // logical tiles [x*r, (x+1)*r), r = ceil(nreal / 8), all run on XCD x, so
@@ -211,53 +224,79 @@ __device__ __forceinline__ bool gg_tile(const int* __restrict__ offs,
   // leaves the bound's surplus on the last XCD and up to a round more on the
   // others: the T = 2048 shared down projection, 256 tiles, took 305 us.)
   // Logical tiles are numbered group by group: group g owns
-  // [gstart * n_tiles, (gstart + mtg) * n_tiles), gstart = tile_start[g].
+  // [gstart * n_tiles, (gstart + mtg) * n_tiles), gstart = tile_start[g]; with
+  // runs a short group has as many as it has runs.
   const unsigned b = blockIdx.x;
   const int lane0 = threadIdx.x & 63;
+  const bool runs = RUN && G <= kScanG;
+  // row tiles of rows [lo, hi); with runs also, in the upper half, whether the group is
+  // short
+  auto tiles_of = [&](int lo, int hi) -> int {
+    return (hi - lo + BM - 1) / BM + (runs && hi > lo && hi - lo <= 128 ? 1 << 16 : 0);
+  };
   // total row tiles: from the plan (G > kScanG) or a scan of the group ends
-  int total_rt = 0, incl0 = 0, tiles0 = 0;  // incl0 / tiles0: groups 0..63, lane = group
+  int total_rt = 0;
+  int lo0 = 0, hi0 = 0, incl0 = 0, tiles0 = 0;  // groups 0..63, lane = group
   if (G <= kScanG) {
     for (int base = 0; base < G; base += 64) {
-      const int t = group_tiles(offs, base + lane0, G, M, BM);
+      int lo, hi;
+      group_rows(offs, base + lane0, G, M, lo, hi);
+      const int t = tiles_of(lo, hi);
       const int incl = wave_incl_scan(t);
       if (base == 0) {
+        lo0 = lo;
+        hi0 = hi;
         incl0 = incl;
         tiles0 = t;
       }
-      total_rt += __shfl(incl, 63, 64);
+      total_rt += __builtin_amdgcn_readlane(incl, 63);
     }
   } else {
-    total_rt = tile_start[G];
+    total_rt = __builtin_amdgcn_readfirstlane(tile_start[G]);
   }
-  total_rt = __builtin_amdgcn_readfirstlane(total_rt);  // wave-uniform: keep it in an SGPR
-  const unsigned nreal = (unsigned)total_rt * (unsigned)n_tiles;
+  int log = 0;
+  unsigned nreal;
+  if (runs) {
+    log = gg_run(total_rt & 0xffff, total_rt >> 16, n_tiles, KT, (int)gridDim.x);
+    nreal = gg_blocks(total_rt & 0xffff, total_rt >> 16, n_tiles, log);
+  } else {
+    nreal = (unsigned)total_rt * (unsigned)n_tiles;
+  }
   const unsigned r = (nreal + 7u) >> 3;
   if ((b >> 3) >= r) return false;
   const unsigned l = (b & 7u) * r + (b >> 3);
   if (l >= nreal) return false;
-  const int lt = (int)(l / (unsigned)n_tiles);
-  // group g of row tile lt: gstart <= lt < gstart + mtg (the first group whose
-  // inclusive tile count exceeds lt; groups without tiles never qualify)
-  int g = 0, gstart = 0, mtg = 0;
+  // group g of logical tile l: the first group whose inclusive count of logical tiles
+  // exceeds l (groups without tiles never qualify); lt, and the counts compared with
+  // it, are row tiles without runs
+  const int lt = runs ? (int)l : (int)(l / (unsigned)n_tiles);
+  auto count = [&](int t) { return runs ? gg_blocks(t & 0xffff, t >> 16, n_tiles, log) : t; };
+  int g = 0, gstart = 0, mtg = 0, gs = 0, ge = 0;
   if (G <= 64) {
-    const unsigned long long m = __ballot(lane0 < G && incl0 > lt);
+    const unsigned long long m = __ballot(lane0 < G && count(incl0) > lt);
     g = __ffsll((long long)m) - 1;
-    mtg = __shfl(tiles0, g, 64);
-    gstart = __shfl(incl0, g, 64) - mtg;
+    mtg = __builtin_amdgcn_readlane(tiles0, g);
+    gstart = __builtin_amdgcn_readlane(incl0, g) - mtg;
+    gs = __builtin_amdgcn_readlane(lo0, g);
+    ge = __builtin_amdgcn_readlane(hi0, g);
   } else if (G <= kScanG) {
     int carry = 0;
     for (int base = 0; base < G; base += 64) {
-      const int t = group_tiles(offs, base + lane0, G, M, BM);
+      int lo, hi;
+      group_rows(offs, base + lane0, G, M, lo, hi);
+      const int t = tiles_of(lo, hi);
       const int incl = wave_incl_scan(t) + carry;
-      const unsigned long long m = __ballot(base + lane0 < G && incl > lt);
+      const unsigned long long m = __ballot(base + lane0 < G && count(incl) > lt);
       if (m) {
         const int L = __ffsll((long long)m) - 1;
         g = base + L;
-        mtg = __shfl(t, L, 64);
-        gstart = __shfl(incl, L, 64) - mtg;
+        mtg = __builtin_amdgcn_readlane(t, L);
+        gstart = __builtin_amdgcn_readlane(incl, L) - mtg;
+        gs = __builtin_amdgcn_readlane(lo, L);
+        ge = __builtin_amdgcn_readlane(hi, L);
         break;
       }
-      carry = __shfl(incl, 63, 64);
+      carry = __builtin_amdgcn_readlane(incl, 63);
     }
   } else {
     // the last g with tile_start[g] <= lt
@@ -266,30 +305,33 @@ __device__ __forceinline__ bool gg_tile(const int* __restrict__ offs,
       const int mid = (lo + hi + 1) >> 1;
       if (tile_start[mid] <= lt) lo = mid; else hi = mid - 1;
     }
-    g = lo;
-    gstart = tile_start[g];
-    mtg = tile_start[g + 1] - gstart;
+    g = __builtin_amdgcn_readfirstlane(lo);
+    gstart = __builtin_amdgcn_readfirstlane(tile_start[g]);
+    mtg = __builtin_amdgcn_readfirstlane(tile_start[g + 1]) - gstart;
+    group_rows(offs, g, G, M, gs, ge);
   }
-  // wave-uniform results of shuffles: SGPRs, not VGPRs the K loop needs
-  g = __builtin_amdgcn_readfirstlane(g);
-  gstart = __builtin_amdgcn_readfirstlane(gstart);
-  mtg = __builtin_amdgcn_readfirstlane(mtg);
+  int li = (int)l - (runs ? count(gstart) : gstart * n_tiles);
+  const int rlast = ge - 1;  // last row of the group
+  const bool ident = ident_m > 0 && ge - gs == ident_m;
+  if (runs && mtg >> 16) {  // a run of a short group
+    const int nt = li << log, nt1 = min((li + 1) << log, n_tiles);
+    // Blocks start at different tiles of their runs: those that run together would
+    // else all be at even tiles, whose addresses share memory channels (128 experts of
+    // 4096 x 2048: 1022 us for 727).
+    out = GgTile{g, gs, gs, rlast, nt, nt1, nt1 - nt == 2 ? li & 1 : 0, ident};
+    return true;
+  }
   // Inside a group, column blocks of kSuperN n-tiles, row tiles across each
   // block, n fastest: 32 consecutive tiles (one XCD's co-running blocks) are
   // 4 row tiles x 8 weight tiles, so each A slice and each weight slice of a
   // K step is fetched from HBM once and then reused from that XCD's L2.
   constexpr int kSuperN = 8;
-  const int li = (int)l - gstart * n_tiles;
   const int nblk = li / (mtg * kSuperN);
   const int rem = li - nblk * mtg * kSuperN;
   const int ncols = min(kSuperN, n_tiles - nblk * kSuperN);
   const int mt_local = rem / ncols;
   const int nt = nblk * kSuperN + rem % ncols;
-  const int gs = g > 0 ? min(max(offs[g - 1], 0), M) : 0;
-  const int ge = min(max(offs[g], 0), M);
-  const int r0 = gs + mt_local * BM;               // first row of the tile
-  const int rlast = ge - 1;                        // last row of the group
-  out = GgTile{g, gs, r0, rlast, nt, ident_m > 0 && ge - gs == ident_m};
+  out = GgTile{g, gs, gs + mt_local * BM, rlast, nt, nt + 1, 0, ident};
   return true;
 }
 
@@ -312,11 +354,11 @@ template <GgType TY> __device__ constexpr int a_at(int buf, int x) {
 }
 __device__ constexpr int raw_at(int buf, int x) { return 6 * kHalf + (buf * 2 + x) * kRaw; }
 __device__ constexpr int sc_at(int buf, int x) { return 8 * kHalf + (buf * 2 + x) * 2048; }
-// bf16 / int8 tiles of at most 128 rows: stages of B0, B1 and 128 or 64 rows of A
-constexpr int kShort128 = 3 * kHalf, kShort64 = 2 * kHalf + kHalf / 2;
+// bf16 / int8 tiles of at most 128 rows: stages of B0, B1 and up to 128 rows of A
+constexpr int kStages = 3, kRunMax = 2;
 template <GgType TY, bool SHORT>
-constexpr int kLds = TY == kFp8 ? 8 * kHalf + 8192 : SHORT ? 4 * kShort64 : 8 * kHalf;
-static_assert(4 * kShort64 >= 8 * kHalf && 4 * kShort64 >= 3 * kShort128, "LDS map");
+constexpr int kLds = TY == kFp8 ? 8 * kHalf + 8192 : SHORT ? kStages * 3 * kHalf : 8 * kHalf;
+static_assert(kStages * 3 >= 8, "LDS map");
 
 template <int N>
 __device__ __forceinline__ void wait_vm() {
@@ -350,12 +392,15 @@ __global__ __launch_bounds__(512) void grouped_gemm_kernel(
   constexpr int BM = kGgBM;
   __shared__ __attribute__((aligned(1024))) char lds[kLds<TY, SHORT>];
   GgTile tile;
-  if (!gg_tile<BM>(offs, tile_start, G, M, n_tiles, ident_m, tile)) return;
+  const int KT = K * EL / 128;
+  if (!gg_tile<BM, SHORT>(offs, tile_start, G, M, n_tiles, KT, ident_m, tile)) return;
   // wave-uniform: in SGPRs
   const int g = __builtin_amdgcn_readfirstlane(tile.g), gs = __builtin_amdgcn_readfirstlane(tile.gs);
   const int r0 = __builtin_amdgcn_readfirstlane(tile.r0);
   const int rlast = __builtin_amdgcn_readfirstlane(tile.rlast);
   const int nt = __builtin_amdgcn_readfirstlane(tile.nt);
+  const int nt1 = __builtin_amdgcn_readfirstlane(tile.nt1);
+  const int rot = __builtin_amdgcn_readfirstlane(tile.rot);
   const bool ident = tile.ident;
 
   const int lane = threadIdx.x & 63;
@@ -369,14 +414,17 @@ __global__ __launch_bounds__(512) void grouped_gemm_kernel(
   // weight rows past N are loaded (clamped), never stored.
   // B half y, instruction q of this wave: rows (wave*2 + q)*8 .. +8 of the half
   const char* bsrc[2][2];
+  auto set_b = [&](int nt) __attribute__((always_inline)) {
 #pragma unroll
-  for (int y = 0; y < 2; ++y)
+    for (int y = 0; y < 2; ++y)
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int r = (wave * 2 + q) * 8 + lane / 8, c = (lane & 7) ^ swz(r);
-      const int wrow = SWIGLU ? nt * 128 + r : nt * 256 + y * 128 + r;
-      bsrc[y][q] = (SWIGLU && y ? w1 : w0) + ((long long)g * N + min(wrow, N - 1)) * rowb + c * 16;
-    }
+      for (int q = 0; q < 2; ++q) {
+        const int r = (wave * 2 + q) * 8 + lane / 8, c = (lane & 7) ^ swz(r);
+        const int wrow = SWIGLU ? nt * 128 + r : nt * 256 + y * 128 + r;
+        bsrc[y][q] =
+            (SWIGLU && y ? w1 : w0) + ((long long)g * N + min(wrow, N - 1)) * rowb + c * 16;
+      }
+  };
   // A half x: as B.  fp8: one instruction of 16 rows x 64 bytes, wave*16 .. +16, in
   // lane order (only this wave reads it), and the index of the lane's row scale
   // from the tile's first (fewer than 2^31 scales in all)
@@ -491,18 +539,46 @@ __global__ __launch_bounds__(512) void grouped_gemm_kernel(
     barrier();
   };
 
-  const int KT = K * EL / 128;
   const int rows = rlast + 1 - r0;  // of this tile, 256 if more
-  // A tile of at most RA = 128 or 64 rows (a small group, or a group's last tile):
-  // the loads bound it, so all waves step together through a ring of NB stages of
-  // RA rows of A and the 256 weight rows, one barrier a step, NB - 1 steps in
-  // flight.  The same wave -> row and column map, so the waves of rows past RA
-  // (and the second row half) have nothing to multiply.
-  auto short_loop = [&]<int RA, int NB>(std::integral_constant<int, RA>,
-                                        std::integral_constant<int, NB>)
-                        __attribute__((always_inline)) {
-    constexpr int STAGE = 2 * kHalf + RA * 128;
-    const bool loads_a = wave * 16 < RA;
+  // The block's column tiles over at most RA = 128 or 64 rows (a small group, or a
+  // group's last tile): the loads bound them, so all waves step together through a
+  // ring of three stages of RA rows of A and the 256 weight rows, one barrier a step,
+  // two steps in flight, also across the end of a tile.  A wave has RA / 2 rows and
+  // 64 weight rows (SwiGLU: 32 of each half).  Only 16-row blocks that hold rows are
+  // loaded, read, multiplied and stored.  The MFMA operands are swapped, so a lane
+  // ends with four neighbouring columns of a row (column fc*4 + e, row fr of a
+  // 16 x 16 block); two column blocks exchanged between lanes make 16-byte stores, 64
+  // bytes of a row per instruction.
+  auto short_run = [&]<int RA>(std::integral_constant<int, RA>) __attribute__((always_inline)) {
+    constexpr int NB = kStages, STAGE = 2 * kHalf + RA * 128, NI = RA / 32, NY = SWIGLU ? 1 : 2;
+    constexpr int OUTC = SWIGLU ? 128 : 256;
+    const int wr = wm * (RA / 2), wc = wn * (SWIGLU ? 32 : 64);
+    constexpr int YB = SWIGLU ? 128 : 32;  // B rows between the wave's two blocks y
+    const int nb = min(max((rows - wr + 15) >> 4, 0), NI);  // this wave's blocks with rows
+    const int len = nt1 - nt, S = KT * len;
+    auto tile_at = [&](int j) { return nt + (j + rot >= len ? j + rot - len : j + rot); };
+    // int8: the row scale of row fr, the column scales of column fr for every tile
+    float rs[NI], cs[kRunMax][2][2];
+    if constexpr (I8) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int row = min(r0 + wr + i * 16 + fr, rlast);
+        rs[i] = ident ? ex.ident[row - gs] : ex.a[ex.a_idx ? ex.a_idx[row] : row];
+      }
+#pragma unroll
+      for (int c = 0; c < kRunMax; ++c)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const int col =
+                tile_at(min(c, len - 1)) * OUTC + (SWIGLU ? 0 : y * 32) + wc + j * 16 + fr;
+            cs[c][y][j] = (SWIGLU && y ? ex.w1 : ex.w0)[(long long)g * N + min(col, N - 1)];
+          }
+    }
+    const bool loads_a = wave * 16 < rows;
+    int kin = 0, jin = 0;  // K step and tile of the next issue
+    set_b(tile_at(0));
     auto issue = [&](int st) __attribute__((always_inline)) {
       char* d = lds + st * STAGE + wave * 2048;
 #pragma unroll
@@ -519,52 +595,152 @@ __global__ __launch_bounds__(512) void grouped_gemm_kernel(
           asrc[0][q] += 128;
         }
       }
+      if (++kin == KT) {
+        kin = 0;
+        set_b(tile_at(++jin));
+#pragma unroll
+        for (int q = 0; q < NA; ++q) asrc[0][q] -= rowb;
+      }
     };
-    int st_in = 0, st = 0;
-    for (; st_in < NB - 1 && st_in < KT; ++st_in) issue(st_in);
-    st_in = NB - 1;
-    for (int kt = 0; kt < KT; ++kt) {
-      // this wave's part of the step landed once at most NB - 2 later ones are
-      // outstanding; the barrier makes that true for every wave, and every wave is
-      // past its reads of the stage refilled now
-      if (kt + NB - 2 >= KT) wait_vm<0>();
-      else if (loads_a) wait_vm<(NB - 2) * 6>();
-      else wait_vm<(NB - 2) * 4>();
+    // a run shorter than the ring: the stages past it are loaded (weight rows are
+    // clamped) and not read
+#pragma unroll
+    for (int q = 0; q < NB - 1; ++q) issue(q);
+    int st_in = NB - 1, st = 0;
+    if constexpr (I8) {  // the scales are here before the loop's own waits begin
+#pragma unroll
+      for (int i = 0; i < NI; ++i) asm volatile("" : "+v"(rs[i]));
+#pragma unroll
+      for (int c = 0; c < kRunMax; ++c)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) asm volatile("" : "+v"(cs[c][y][j]));
+    }
+    int ao[2], bo[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const int c = ((kk * 4 + fc) ^ swz(fr)) * 16;
+      ao[kk] = 2 * kHalf + (wr + fr) * 128 + c;
+      bo[kk] = (wc + fr) * 128 + c;
+    }
+    auto product = [&](int y, int i, int j, int e) -> float {
+      if constexpr (I8)
+        return (float)acc[0][y][i][j][e] * (rs[i] * __shfl(cs[0][y][j], fc * 4 + e, 64));
+      else
+        return acc[0][y][i][j][e];
+    };
+    int kt = 0, jt = 0;
+    for (int u = 0; u < S; ++u) {
+      // this wave's part of the step landed once at most the next one is outstanding
+      // (stores count too: then it waits for more); the barrier makes that true for
+      // every wave, and every wave is past its reads of the stage refilled now
+      const int rem = S - 1 - u;
+      if (rem == 0) wait_vm<0>();
+      else if (loads_a) wait_vm<6>();
+      else wait_vm<4>();
       barrier();
-      if (kt + NB - 1 < KT) issue(st_in);
-      if (live0) {
-        const char* p = lds + st * STAGE;
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            fa[kk][i] = *reinterpret_cast<const bf16x8*>(p + 2 * kHalf + aoff[kk] + i * 2048);
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            fb0[0][kk][j] = *reinterpret_cast<const bf16x8*>(p + boff[kk] + j * 2048);
-            fb1[kk][j] = *reinterpret_cast<const bf16x8*>(p + kHalf + boff[kk] + j * 2048);
-          }
-        }
+      if (rem >= NB - 1) issue(st_in);
+      const char* p = lds + st * STAGE;
+      if (nb > 0) {
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-          for (int y = 0; y < 2; ++y)
+          for (int j = 0; j < 2; ++j) {
+            fb0[0][kk][j] = *reinterpret_cast<const bf16x8*>(p + bo[kk] + j * 2048);
+            fb1[kk][j] = *reinterpret_cast<const bf16x8*>(p + YB * 128 + bo[kk] + j * 2048);
+          }
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < NI; ++i) {
+          if (i >= nb) break;
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk)
+            fa[kk][i] = *reinterpret_cast<const bf16x8*>(p + ao[kk] + i * 2048);
+        }
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          if (i >= nb) break;
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
 #pragma unroll
               for (int j = 0; j < 2; ++j)
                 acc[0][y][i][j] =
-                    mfma_step<I8>(fa[kk][i], y ? fb1[kk][j] : fb0[0][kk][j], acc[0][y][i][j]);
+                    mfma_step<I8>(y ? fb1[kk][j] : fb0[0][kk][j], fa[kk][i], acc[0][y][i][j]);
+        }
       }
       st = st == NB - 1 ? 0 : st + 1;
       st_in = st_in == NB - 1 ? 0 : st_in + 1;
+      if (++kt < KT) continue;
+      kt = 0;  // the tile is complete
+      const int c0 = tile_at(jt++) * OUTC + wc;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        if (i >= nb) break;
+        const int rl = wr + i * 16 + fr;
+        unsigned short* o = out + (long long)(r0 + rl) * N;
+#pragma unroll
+        for (int y = 0; y < NY; ++y) {
+          unsigned short v[2][4];
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              v[j][e] = (unsigned short)f2bf(
+                  SWIGLU ? swiglu(product(0, i, j, e), product(1, i, j, e)) : product(y, i, j, e));
+          if ((N & 7) == 0) {
+            // lanes of odd fc give column block 0 and take column block 1
+            u32x4 pk;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const auto sw = __builtin_amdgcn_permlane16_swap(
+                  (unsigned)v[0][2 * h] | (unsigned)v[0][2 * h + 1] << 16,
+                  (unsigned)v[1][2 * h] | (unsigned)v[1][2 * h + 1] << 16, false, false);
+              pk[h] = sw[0];
+              pk[2 + h] = sw[1];
+            }
+            const int col = c0 + y * 32 + (fc & 1) * 16 + (fc >> 1) * 8;
+            if (rl < rows && col < N) *reinterpret_cast<u32x4*>(o + col) = pk;
+          } else {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const int col = c0 + y * 32 + j * 16 + fc * 4 + e;
+                if (rl < rows && col < N) o[col] = v[j][e];
+              }
+          }
+        }
+      }
+#pragma unroll
+      for (int y = 0; y < 2; ++y)
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[0][y][i][j] = AccV{0, 0, 0, 0};
+      if constexpr (I8) {
+#pragma unroll
+        for (int c = 0; c + 1 < kRunMax; ++c)
+#pragma unroll
+          for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) cs[c][y][j] = cs[c + 1][y][j];
+      }
     }
   };
-  if (SHORT && rows <= 64) {
-    if constexpr (SHORT) short_loop(std::integral_constant<int, 64>{}, std::integral_constant<int, 4>{});
-  } else if (SHORT && rows <= 128) {
-    if constexpr (SHORT) short_loop(std::integral_constant<int, 128>{}, std::integral_constant<int, 3>{});
-  } else {
+  if constexpr (SHORT) {
+    if (rows <= 64) {
+      short_run(std::integral_constant<int, 64>{});
+      return;
+    }
+    if (rows <= 128) {
+      short_run(std::integral_constant<int, 128>{});
+      return;
+    }
+  }
+  {
+    set_b(nt);
     issue_b(0, 0);
     issue_a(0, 0);
     if constexpr (F8) issue_s(0, 0);
@@ -757,14 +933,22 @@ static hipError_t launch_gg(const void* a, const void* ident_a, int ident_m, con
   }
   if (M == 0 || N == 0 || G == 0) return hipSuccess;
   const int n_tiles = grouped_gemm_n_tiles(N, swiglu);
-  const long long blocks = (((long long)M + kGgBM - 1) / kGgBM + G) * n_tiles;
-  const dim3 grid((unsigned)((blocks + 7) / 8 * 8)), blk(512);
   // Groups of at most 128 rows on average: the kernel with the ring loop for short
   // tiles.  The one without it keeps 0.3 .. 0.6% at T = 8192 (whole layer 10.31 /
-  // 10.36 ms; it needs 256 registers and 160 KB of LDS), the one with it gains 2.8%
-  // at T = 16 (1671 / 1625 us).
+  // 10.36 ms; it needs 256 registers).
   constexpr bool kRing = TY != kFp8;
+  constexpr int EL = TY == kInt8 ? 1 : 2;
   const bool ring = kRing && (long long)M <= 128ll * G;
+  // Runs are chosen here as if the rows reached groups at random and all were short, and
+  // again by every block for the real counts, as far as this grid holds them.  Above 96
+  // rows on average some random group is long: its blocks would open another round of
+  // two-tile ones (bf16, 128 experts, 1024 x 1024, 100 rows: 64 / 86 us).
+  const int reach = (int)(G * (1.0 - std::exp(-(double)M / G)) + 0.5);
+  const int log = ring && G <= kScanG && (long long)M <= 96ll * G
+                      ? gg_run(reach, reach, n_tiles, K * EL / 128, 0x7fffffff)
+                      : 0;
+  const long long blocks = gg_grid(M, G, n_tiles, log);
+  const dim3 grid((unsigned)((blocks + 7) / 8 * 8)), blk(512);
 #define MOE_GG(SW, SH)                                                                         \
   hipLaunchKernelGGL((grouped_gemm_kernel<SW, TY, SH>), grid, blk, 0, s, (const char*)a,        \
                      (const char*)ident_a, ident_m, (const char*)w0,                           \
