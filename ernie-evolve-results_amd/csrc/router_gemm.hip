@@ -82,6 +82,7 @@ __global__ __launch_bounds__(64 * WM * WN) void router_gemm_dma_kernel(
   const int wm = wave / WN, wn = wave % WN;
   const long long m0 = (long long)blockIdx.x * BM;
   const int n0 = blockIdx.y * BN;
+  if (BN == 64 && m0 >= T) return;  // the grid's rounding
   // K partition z of gridDim.z: whole 64-wide steps, as even as they go
   const int U = H / BK, z = blockIdx.z, nz = gridDim.z;
   const int kb = (int)((long long)z * U / nz) * BK;
@@ -176,7 +177,14 @@ __global__ __launch_bounds__(64 * WM * WN) void router_gemm_dma_kernel(
 template <int BM, int BN, int NS, int WM, int WN>
 static hipError_t launch_dma(const __bf16* x, const __bf16* w, int T, int H, int N, int ksplit,
                              float* out, hipStream_t s) {
-  const dim3 grid((unsigned)((T + BM - 1) / BM), (unsigned)((N + BN - 1) / BN), (unsigned)ksplit);
+  // 64 columns: the row tiles are rounded up to a multiple of 8, so that the column tiles
+  // of a row tile run on one XCD, whose L2 serves x to all of them (128 x 64 tiles, route
+  // in us: E = 128, H = 4096, T = 15000, 118 row tiles, 46 / 37; E = 256, H = 4096,
+  // T = 8000, 63 row tiles, 50 / 37).  The wider tiles read x once or twice and gain
+  // nothing (128 x 128, E = 256, H = 1024, T = 9000: 21.6 / 22.9).
+  const int mt = (T + BM - 1) / BM, ny = (N + BN - 1) / BN;
+  const dim3 grid((unsigned)(BN == 64 && ny > 1 ? (mt + 7) / 8 * 8 : mt), (unsigned)ny,
+                  (unsigned)ksplit);
   hipLaunchKernelGGL((router_gemm_dma_kernel<BM, BN, NS, WM, WN>), grid, dim3(64 * WM * WN), 0,
                      s, x, w, T, H, N, out, N * ksplit);
   return hipGetLastError();

@@ -247,8 +247,10 @@ const Tile kTilesF32[] = {{16, 16, launch_wk<16, 16, 8, 2, true>},
 constexpr int kCUs = 256;
 
 // The tile of the least operand bytes per CU: rounds of blocks x operand rows
-// per block (an fp32 weight row counts twice).  Measured over T = 1 .. 16384 at
-// E = 32 .. 256, H = 512 .. 8192 it picks the fastest tile or one within 5% of it.
+// per block (an fp32 weight row counts twice).  Measured for the GEMM alone over
+// T = 1 .. 16384, E = 32 .. 256, H = 512 .. 8192: at 349 of 360 points the fastest tile
+// or one within 5% of it, at worst 22% behind (E = 256, H = 8192, T = 10000: 128 x 128
+// 69 us, 80 x 64 57).
 static const Tile* pick(int T, int E, bool wf32) {
   const Tile* t = wf32 ? kTilesF32 : kTiles;
   const int n = (int)(wf32 ? sizeof(kTilesF32) : sizeof(kTiles)) / (int)sizeof(Tile);
@@ -274,10 +276,18 @@ static const Tile* pick(int T, int E, bool wf32) {
 //   elsewhere, against K split over blocks with the partial sums added by the
 //     scoring kernel: that path moves fewer operand bytes (larger tiles) but
 //     writes and reads the partials, so it wins for long rows and many tokens:
-//     E = 256, H = 4096 T = 12000 74 / 64, 16384 73 / 70, 32768 118 / 167;
-//     E = 64, H = 8192 T = 2500 20.4 / 19.0, 3000 23.0 / 25.9; E = 128,
-//     H = 7168 T = 3000 28.0 / 27.8, 4096 30.4 / 33.1 -- and at E = 128 from
-//     T = 10000 on the 128 x 128 tile beats its 64-row tiles (72 / 56).
+//     E = 256, H = 4096 T = 4500 32 / 25, 6000 31 / 34, 7000 49 / 35, 10100 40 / 47,
+//     12200 53 / 50, 32768 91 / 120; H = 2048 T = 12200 44 / 32; E = 64, H = 8192
+//     T = 900 13.8 / 12.5, 2300 17.3 / 17.5, 2800 18.2 / 18.0.
+//   E = 128 above 8192 tokens, where that path has one tile of 64 tokens and all
+//     experts per 64 tokens and no K split: the 80 x 64 tiles up to 10240 (H = 4096
+//     T = 9000 32 / 26).  From there the tiles are 128 x 64, above 16384 128 x 128.
+//     They have the same operand bytes per CU (up to 16384 tokens) and lose while x
+//     stays in the 256 MB memory-side cache, except where H is short (H = 1024
+//     T = 12200 20.8 / 17.8, 25000 23.3 / 23.9; H = 4096 T = 12200 33.5 / 34.9, 22000
+//     47 / 49; H = 8192 T = 11000 49 / 57), and win beyond (H = 8192 T = 15000 74 / 61,
+//     18000 125 / 93; H = 7168 T = 32768 140 / 115) unless the last of the 128-token
+//     rounds is nearly empty (H = 8192 T = 45000 216 / 231).
 //   fp32 weights: E = 64, H = 8192 T = 3000 32.7 / 28.9, 4096 34.9 / 42.0;
 //     E = 256, H = 4096 T = 700 30 / 19, 4096 42 / 61; E = 32, H = 4096
 //     T = 6000 22.9 / 20.0, 8192 27.9 / 29.1.
@@ -286,7 +296,12 @@ bool router_wk_use(int T, int H, int E, bool wf32) {
   if (wf32) return (long long)T * E <= (H <= 4096 ? 229376 : 196608);
   if (E == 256 && H == 7168) return T <= 16384;
   if (E == 128 && H == 2048) return T <= 10240;
-  if (E == 128 && T > 8192) return true;
+  if (E == 128 && T > 8192) {
+    if (T <= 10240 || (H <= 2048 && T <= 16384)) return true;
+    if ((long long)T * H <= 110ll << 20) return false;
+    const int r = (T + 16383) / 16384;  // rounds of 64-token tiles, half as many of 128
+    return r == 1 || 5 * ((r + 1) / 2) < 3 * r;
+  }
   return H <= 4096 ? T <= 12288 : (long long)T * H <= 2560ll * 8192;
 }
 

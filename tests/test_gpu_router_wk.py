@@ -48,6 +48,25 @@ def test_logits(cuda, E, H, T, fp32):
         assert_logits(M.router_gemm(x, w), x, w, False)
 
 
+# (E, H, T): the 128 x 64 tiles with 41, 81, 82 and 127 row tiles (the grid rounds them up
+# to a multiple of 8), the 128 x 128 tiles, and E = 128 either side of each line of the rule
+LARGE = [(256, 1024, 5121), (256, 4096, 8065), (128, 1024, 10241), (128, 1024, 10369),
+         (128, 1024, 16256), (256, 1024, 8193), (256, 1024, 12001), (128, 8192, 16385),
+         (128, 1024, 10240), (128, 4096, 10241), (128, 1024, 16385), (128, 8192, 32769)]
+
+
+@pytest.mark.parametrize("E,H,T", LARGE)
+def test_large_batches(cuda, E, H, T):
+    print("router_wk large E=%d H=%d T=%d" % (E, H, T), flush=True)
+    x, w = inputs(T, H, E, T + H, cuda)
+    w = w.bfloat16()
+    logits, ids, wts, counts = M.route(x, w, None, 8, RouteCfg())
+    for lo in range(0, T, 8192):  # the float64 copies a piece at a time
+        assert_logits(logits[lo:lo + 8192], x[lo:lo + 8192], w, False)
+    i2, w2, c2 = M.topk(logits, None, 8, RouteCfg())
+    assert torch.equal(ids, i2) and torch.equal(wts, w2) and torch.equal(counts, c2)
+
+
 def test_unaligned_logits(cuda):
     """moe_router_gemm takes logits at any 4-byte address."""
     T, H, E = 33, 1024, 64
