@@ -519,9 +519,16 @@ int moe_route_permute(const void* x, const void* w, int w_dtype, const float* bi
   // whole permute blocks, it writes the permute's block histograms and the
   // histogram launch is skipped.  The route never writes counts here: the
   // index kernel writes them from the scanned totals.
-  // Few pairs: the permute counts them itself in its one launch.
-  const bool small = xg && moe::small_permute_use(T, H, k, 2, out_dtype == MOE_DTYPE_FP8E4M3FN);
-  const RouteHist handoff = small ? kHistNone : route_block_hist(T, H, E, k, w_dtype, cfg);
+  // Few pairs: the permute counts them itself in its one launch -- unless the histograms
+  // would leave the general path two short ones and each block of this launch ranks 40
+  // pairs (8 slots, bf16 rows of under 128 pieces; us, two launches / one: E = 8, H = 640,
+  // T = 106 12.9 / 13.7, T = 16 12.2 / 13.2; E = 16, H = 512, T = 64 11.3 / 12.0; with 4
+  // slots E = 8, H = 640, T = 256 12.4 / 11.2).
+  const bool fp8 = out_dtype == MOE_DTYPE_FP8E4M3FN;
+  RouteHist handoff = route_block_hist(T, H, E, k, w_dtype, cfg);
+  if (xg && moe::small_permute_use(T, H, k, 2, fp8) &&
+      !(handoff != kHistNone && k == 8 && T > 8 && H < 1024 && !fp8))
+    handoff = kHistNone;
   void* stage = (char*)pws + moe_permute_workspace_bytes(T, E, k);
   int32_t* sub = (int32_t*)((char*)pws + moe_permute_fp8_workspace_bytes(T, H, E, k));
   int32_t* hist = handoff == kHistSub ? sub : handoff == kHistBlocks ? (int32_t*)pws : nullptr;

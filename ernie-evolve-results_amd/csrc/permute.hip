@@ -220,21 +220,23 @@ hipError_t launch_gather_fp8(const void* x, const int32_t* pair_row, const int32
 // each on the host, as much on the device).  Here every block finds the rows of its own
 // pairs from all the ids: pair p of expert e goes to row
 //   #{q : (id_q, q) < (e, p)},
-// the stable expert-major order itself.  A thread holds up to kSmallPairs / 256
-// ids as keys id * kSmallPairs + q, so one pair costs one compare, ballot
-// and popcount per 64 ids.  One more block writes offsets and counts.
+// the stable expert-major order itself.  A thread holds IPT ids as keys
+// id * kSmallPairs + q, so one pair costs one compare, ballot and popcount per 64 ids:
+// IPT = 4 up to 1024 pairs, 8 above (E = 32, H = 512, T = 106, k = 8, 848 pairs: 8.7 us
+// with 8, 7.7 with 4).  One more block writes offsets and counts.
 // At most kSmallPairs pairs (half for the shortest rows, whose blocks rank the
 // pairs of five tokens) and rows of at least kSmallRowItems work items.
 // Measured (MI355X, us a call replayed from a graph, histogram + index + gather
 // launches / this one): bf16, E = 256, H = 7168, k = 8: T = 16 8.1 / 5.8, T = 256
 // 13.1 / 8.9; E = 8, H = 4096, k = 2: T = 64 7.5 / 3.2, T = 1024 9.9 / 6.6; fp8,
 // E = 256, H = 7168, k = 8, T = 128 15.4 / 6.9.  At 2048 pairs and H = 512 the
-// launch would tie the index and gather launches after a histogram handoff.
+// launch would tie the index and gather launches after a histogram handoff; with 8
+// slots and rows of under 128 items it loses to them (moe_route_permute keeps these).
 // ---------------------------------------------------------------------------
 constexpr int kSmallPairs = 2048, kSmallRowItems = 64;
 constexpr int kSmallTok = 256 / kSmallRowItems + 1;  // tokens a block's items touch, at most
 
-template <int K, bool FP8>
+template <int K, bool FP8, int IPT>
 __global__ __launch_bounds__(256) void small_permute_kernel(
     const u32x4* __restrict__ x, const int* __restrict__ ids, int npairs, int E, int k_rt,
     int total, int per_row, u32x4* __restrict__ xg, float* __restrict__ scales,
@@ -244,7 +246,6 @@ __global__ __launch_bounds__(256) void small_permute_kernel(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nb = (int)gridDim.x - (offsets || counts ? 1 : 0);  // gather blocks
-  constexpr int IPT = kSmallPairs / 256;
   int key[IPT];  // ids in (expert, pair) order; invalid ids and places past the end last
 #pragma unroll
   for (int j = 0; j < IPT; ++j) {
@@ -332,22 +333,25 @@ hipError_t launch_small_permute(const void* x, int elem_bytes, bool fp8, const i
                                 hipStream_t s) {
   const int per_row = fp8 ? H / 16 : (int)((long long)H * elem_bytes / 16);
   const int total = T * per_row;  // < 2^31, checked by the caller
+  constexpr int kIpt = kSmallPairs / 256;
+  const bool half = T * k <= kSmallPairs / 2;
   const dim3 grid((unsigned)((total + 255) / 256 + (offsets || counts ? 1 : 0))), blk(256);
-#define MOE_SMALL(KK)                                                                         \
-  {                                                                                           \
-    if (fp8)                                                                                  \
-      hipLaunchKernelGGL((small_permute_kernel<KK, true>), grid, blk, 0, s, (const u32x4*)x, ids, \
-                         T * k, E, k, total, per_row, (u32x4*)xg, scales, row_token, pair_row, \
-                         offsets, counts);                                                    \
-    else                                                                                      \
-      hipLaunchKernelGGL((small_permute_kernel<KK, false>), grid, blk, 0, s, (const u32x4*)x, ids, \
-                         T * k, E, k, total, per_row, (u32x4*)xg, scales, row_token, pair_row, \
-                         offsets, counts);                                                    \
+#define MOE_SMALL_K(KK, F8, IPT)                                                               \
+  hipLaunchKernelGGL((small_permute_kernel<KK, F8, IPT>), grid, blk, 0, s, (const u32x4*)x, ids, \
+                     T * k, E, k, total, per_row, (u32x4*)xg, scales, row_token, pair_row,     \
+                     offsets, counts)
+#define MOE_SMALL(KK)                                    \
+  {                                                      \
+    if (fp8 && half) MOE_SMALL_K(KK, true, kIpt / 2);    \
+    else if (fp8) MOE_SMALL_K(KK, true, kIpt);           \
+    else if (half) MOE_SMALL_K(KK, false, kIpt / 2);     \
+    else MOE_SMALL_K(KK, false, kIpt);                   \
   }
   if (k == 8) MOE_SMALL(8)
   else if (k == 2) MOE_SMALL(2)
   else MOE_SMALL(0)
 #undef MOE_SMALL
+#undef MOE_SMALL_K
   return hipGetLastError();
 }
 

@@ -136,6 +136,15 @@ CASES = [
     (8, 2048, 1, 777, False, False),       # eight columns per block
     (8, 4096, 3, 500, False, False),       # no handoff: 256 % 3 != 0
     (16, 2048, 2, 20000, False, True),     # no handoff: 16 x 625 columns > 8192
+    # few pairs of short rows: index and gather after the handoff (8 slots, more than 8
+    # tokens), and either side of that line in one launch
+    (8, 640, 8, 106, False, False),
+    (16, 512, 8, 9, False, False),
+    (8, 768, 8, 128, False, False),
+    (64, 960, 8, 100, False, False),
+    (8, 640, 8, 8, False, False),
+    (16, 512, 4, 256, False, False),
+    (8, 1024, 8, 106, False, False),
     (8, 1024, 2, 512, False, False),       # C1's shape (fp32 weights: the small-E hi/lo route)
 ]
 

@@ -17,6 +17,9 @@ CASES = [
     (129, 8, 64, 512, torch.bfloat16, False),    # one too many: the general path
     (256, 8, 256, 1032, torch.bfloat16, False),  # 2048 pairs, 129 items a row
     (257, 8, 256, 1032, torch.bfloat16, False),  # general path
+    (256, 4, 32, 1024, torch.bfloat16, False),   # 1024 pairs: 4 ids a thread
+    (205, 5, 64, 1032, torch.bfloat16, False),   # 1025: 8
+    (513, 2, 8, 2048, torch.bfloat16, True),
     (682, 3, 1024, 1024, torch.bfloat16, False),
     (1023, 2, 8, 1160, torch.bfloat16, False),
     (100, 6, 40, 260, torch.float32, False),     # 65 items a row
