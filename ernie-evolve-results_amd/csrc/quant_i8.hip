@@ -86,15 +86,16 @@ __global__ __launch_bounds__(kQuantThreads) void quant_rows_i8_kernel(
     __syncthreads();
     Rv = n_grp * group_rows;
   }
-  for (int rb = blockIdx.x * RB; rb < Rv; rb += gridDim.x * RB) {
+  // unsigned: R may be 2^31 - 1, and a block's last step goes up to 2^17 rows past Rv
+  for (unsigned rb = blockIdx.x * RB; rb < (unsigned)Rv; rb += gridDim.x * RB) {
     // RB consecutive (virtual) rows per pass: all their loads are issued together
     bool act[RB];
     int rows[RB];
 #pragma unroll
     for (int i = 0; i < RB; ++i) {
-      const int v = rb + i;
-      act[i] = v < Rv;
-      rows[i] = group_counts ? grp[min(v, Rv - 1) / group_rows] * group_rows + v % group_rows : v;
+      act[i] = rb + i < (unsigned)Rv;
+      const int v = act[i] ? (int)(rb + i) : Rv - 1;
+      rows[i] = group_counts ? grp[v / group_rows] * group_rows + v % group_rows : v;
     }
     float v[RB][NC][16];
 #pragma unroll

@@ -172,3 +172,20 @@ def test_int8_chain_matches_float_product(cuda):
     ref = h.float() @ wd[0].float().t()
     rel = float((y - ref).norm() / ref.norm())
     assert rel < 0.02, rel
+
+
+def test_quant_rows_up_to_int32(cuda):
+    """Row counts near 2^31: a block steps past the last row in 32 bits without coming
+    back to rows before the first (the last step is 2^17 rows)."""
+    R, K, tail = 2 ** 31 - 5, 16, 300
+    if torch.cuda.mem_get_info()[0] < 140 * 2 ** 30:
+        pytest.skip("needs 105 GiB of device memory")
+    x = torch.zeros(R, K, dtype=torch.bfloat16, device=cuda)
+    g = torch.Generator(device=cuda).manual_seed(7)
+    x[-tail:] = torch.randn(tail, K, generator=g, device=cuda).bfloat16()
+    q, s = M.quant_rows_i8(x)
+    qt, st = M.quant_rows_i8(x[-tail:].contiguous())
+    assert torch.equal(q[-tail:], qt) and torch.equal(s[-tail:], st)
+    for lo in (0, 2 ** 30, R - tail - 2 ** 18):  # all-zero rows
+        assert int(q[lo:lo + 2 ** 18 - 1].count_nonzero()) == 0
+        assert int(s[lo:lo + 2 ** 18 - 1].count_nonzero()) == 0
