@@ -250,7 +250,9 @@ static int route_launch(const void* x, const void* w, int w_dtype, const float* 
   // parts == 1: the GEMM writes the logits; else it writes [T, parts*E]
   // partial sums and the scoring kernel adds them and writes the logits.
   float* gout = parts > 1 ? (float*)wsp : logits;
-  rc = launched(moe::launch_router_gemm((const __bf16*)x, wb, T, H, N, ksplit, gout, s),
+  // in chains no longer than with router_gemm_ksplit partitions
+  const int chains = (moe::router_gemm_ksplit(T, H, N) + ksplit - 1) / ksplit;
+  rc = launched(moe::launch_router_gemm((const __bf16*)x, wb, T, H, N, ksplit, chains, gout, s),
                 "router_gemm");
   if (rc) return rc;
   // an fp32 weight's partials fold as (sum of hi) + (sum of lo): negative count
@@ -276,7 +278,7 @@ int moe_router_gemm(const void* x, const void* w, int T, int H, int E, float* lo
     return launched(moe::launch_router_wk((const __bf16*)x, w, false, T, H, E, logits,
                                           (hipStream_t)stream),
                     "router_wk");
-  return launched(moe::launch_router_gemm((const __bf16*)x, (const __bf16*)w, T, H, E, 1, logits,
+  return launched(moe::launch_router_gemm((const __bf16*)x, (const __bf16*)w, T, H, E, 1, 1, logits,
                                           (hipStream_t)stream),
                   "router_gemm");
 }

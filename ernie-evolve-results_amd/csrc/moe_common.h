@@ -50,7 +50,7 @@ namespace moe {
 
 hipError_t launch_wsplit(const float* w, __bf16* wpk, int E, int H, hipStream_t s);
 hipError_t launch_router_gemm(const __bf16* x, const __bf16* w, int T, int H, int N,
-                              int ksplit, float* out, hipStream_t s);
+                              int ksplit, int chains, float* out, hipStream_t s);
 // K partitions: the most a launch uses (sizes the workspace), and those it does.
 int router_gemm_ksplit(int T, int H, int N);
 int router_gemm_ksplit_run(int T, int H, int N);

@@ -64,10 +64,10 @@ hipError_t launch_wsplit(const float* w, __bf16* wpk, int E, int H, hipStream_t 
 //   chunk c of tile row r lives at physical chunk c ^ ((r >> 1) & 7): the 16
 //   rows of one fragment read land on 16 distinct bank groups.
 // ---------------------------------------------------------------------------
-template <int BM, int BN, int NS, int WM, int WN>
+template <int BM, int BN, int NS, int WM, int WN, bool FOLD>
 __global__ __launch_bounds__(64 * WM * WN) void router_gemm_dma_kernel(
     const __bf16* __restrict__ x, const __bf16* __restrict__ w, int T, int H, int N, int kstep,
-    int kmore, float* __restrict__ out, int ldo) {
+    int kmore, int fold, float* __restrict__ out, int ldo) {
   constexpr int BK = 64, CH = 8, ROWB = 128, RPI = 8;
   constexpr int STAGE_B = (BM + BN) * ROWB;
   constexpr int A_INST = BM / RPI, B_INST = BN / RPI, NW = WM * WN;
@@ -118,17 +118,21 @@ __global__ __launch_bounds__(64 * WM * WN) void router_gemm_dma_kernel(
     }
   };
 
-  f32x4 acc[FM][FN];
+  f32x4 acc[FM][FN], tot[FM][FN];  // tot: the chains before this one
+  auto zero = [](f32x4 (&v)[FM][FN]) {
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < FN; ++j) v[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  };
+  zero(acc);
+  zero(tot);
 
 #pragma unroll
   for (int st = 0; st < NS - 1; ++st)
     if (st < KT) issue(st, st);
   const int fr = lane & 15, fc = lane >> 4;
-  for (int kt = 0; kt < KT; ++kt) {
+  auto step = [&](int kt) __attribute__((always_inline)) {
     // This wave's loads of stage kt are done once at most (NS-2) later
     // stages are outstanding; the barrier then publishes every wave's
     // loads and retires the reads of the buffer reloaded next.
@@ -157,6 +161,19 @@ __global__ __launch_bounds__(64 * WM * WN) void router_gemm_dma_kernel(
         for (int j = 0; j < FN; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
     }
+  };
+  if constexpr (FOLD) {
+    for (int kt = 0; kt < KT;) {
+      const int end = min(kt + fold, KT);
+      for (; kt < end; ++kt) step(kt);
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) tot[i][j] += acc[i][j];
+      zero(acc);
+    }
+  } else {
+    for (int kt = 0; kt < KT; ++kt) step(kt);
   }
 
   // partial z of the split-K writes columns [z*N, (z+1)*N) of a row of ldo floats
@@ -169,14 +186,14 @@ __global__ __launch_bounds__(64 * WM * WN) void router_gemm_dma_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const long long row = m0 + wm * WTM + i * 16 + (lane >> 4) * 4 + r;
-        if (row < T && col < N) o[row * ldo + col] = acc[i][j][r];
+        if (row < T && col < N) o[row * ldo + col] = FOLD ? tot[i][j][r] : acc[i][j][r];
       }
     }
 }
 
 template <int BM, int BN, int NS, int WM, int WN>
 static hipError_t launch_dma(const __bf16* x, const __bf16* w, int T, int H, int N, int ksplit,
-                             float* out, hipStream_t s) {
+                             int chains, float* out, hipStream_t s) {
   // 64 columns: the row tiles are rounded up to a multiple of 8, so that the column tiles
   // of a row tile run on one XCD, whose L2 serves x to all of them (128 x 64 tiles, route
   // in us: E = 128, H = 4096, T = 15000, 118 row tiles, 46 / 37; E = 256, H = 4096,
@@ -188,9 +205,24 @@ static hipError_t launch_dma(const __bf16* x, const __bf16* w, int T, int H, int
   // The partitions' bounds are divided here: two 64-bit divisions at the start of every
   // block cost E = 8, H = 640, T = 106 6.0 us a route for 5.8 without, E = 128,
   // H = 7168, T = 16000 73.9 for 66.8.
-  const int U = H / 64;
-  hipLaunchKernelGGL((router_gemm_dma_kernel<BM, BN, NS, WM, WN>), grid, dim3(64 * WM * WN), 0,
-                     s, x, w, T, H, N, U / ksplit, U % ksplit, out, N * ksplit);
+  // A partition is added up in `chains` chains of fp32 sums: an fp32 chain's error grows
+  // with its length, so a call with fewer partitions than it would need for its precision
+  // (router_gemm_ksplit) makes up for it here.  Error against 64 bits, route of E = 256,
+  // H = 4096, T = 8000, whole K: one chain 3.97e-7, four 1.89e-7 (as with 4 partitions);
+  // E = 256, H = 8192, T = 4904, 7 partitions 2.22e-7, two chains in each 1.57e-7 (8
+  // partitions 1.93e-7).
+  const int U = H / 64, fold = ((U + ksplit - 1) / ksplit + chains - 1) / chains;
+#define MOE_DMA(F)                                                                              \
+  hipLaunchKernelGGL((router_gemm_dma_kernel<BM, BN, NS, WM, WN, F>), grid, dim3(64 * WM * WN), \
+                     0, s, x, w, T, H, N, U / ksplit, U % ksplit, fold, out, N * ksplit)
+  if constexpr (BM * BN >= 64 * 128) {  // the smaller tiles always have all their partitions
+    if (chains > 1) {
+      MOE_DMA(true);
+      return hipGetLastError();
+    }
+  }
+  MOE_DMA(false);
+#undef MOE_DMA
   return hipGetLastError();
 }
 
@@ -240,24 +272,27 @@ int router_gemm_ksplit_run(int T, int H, int N) {
 }
 
 // N in {8, 16, 32, 64, 128} or a multiple of 256; H % 64 == 0 (checked by
-// the caller); ksplit at most H / 64.
+// the caller); ksplit at most H / 64, the sum of a partition in `chains` fp32 chains.
 hipError_t launch_router_gemm(const __bf16* x, const __bf16* w, int T, int H, int N, int ksplit,
-                              float* out, hipStream_t s) {
-  if (N >= 256) return launch_dma<256, 128, 3, 4, 4>(x, w, T, H, N, ksplit, out, s);
-  if (N == 128) return launch_dma<64, 128, 3, 1, 4>(x, w, T, H, N, ksplit, out, s);
-  if (N == 64) return launch_dma<64, 64, 3, 2, 2>(x, w, T, H, N, ksplit, out, s);
-  if (N == 32) return launch_dma<64, 32, 3, 4, 1>(x, w, T, H, N, ksplit, out, s);
-  return launch_dma<32, 16, 4, 2, 1>(x, w, T, H, N, ksplit, out, s);
+                              int chains, float* out, hipStream_t s) {
+  if (N >= 256) return launch_dma<256, 128, 3, 4, 4>(x, w, T, H, N, ksplit, chains, out, s);
+  if (N == 128) return launch_dma<64, 128, 3, 1, 4>(x, w, T, H, N, ksplit, chains, out, s);
+  if (N == 64) return launch_dma<64, 64, 3, 2, 2>(x, w, T, H, N, ksplit, chains, out, s);
+  if (N == 32) return launch_dma<64, 32, 3, 4, 1>(x, w, T, H, N, ksplit, chains, out, s);
+  return launch_dma<32, 16, 4, 2, 1>(x, w, T, H, N, ksplit, chains, out, s);
 }
 
-// Whole-K tiles for the batches router_wk.hip gives them (w bf16).
+// Whole-K tiles for the batches router_wk.hip gives them (w bf16), in as many chains as
+// these would have partitions.
 hipError_t launch_router_gemm_128x64(const __bf16* x, const void* w, int T, int H, int N,
                                      float* out, hipStream_t s) {
-  return launch_dma<128, 64, 6, 4, 2>(x, (const __bf16*)w, T, H, N, 1, out, s);
+  return launch_dma<128, 64, 6, 4, 2>(x, (const __bf16*)w, T, H, N, 1,
+                                 router_gemm_ksplit(T, H, N), out, s);
 }
 hipError_t launch_router_gemm_128x128(const __bf16* x, const void* w, int T, int H, int N,
                                       float* out, hipStream_t s) {
-  return launch_dma<128, 128, 5, 2, 4>(x, (const __bf16*)w, T, H, N, 1, out, s);
+  return launch_dma<128, 128, 5, 2, 4>(x, (const __bf16*)w, T, H, N, 1,
+                                 router_gemm_ksplit(T, H, N), out, s);
 }
 
 }  // namespace moe

@@ -12,7 +12,10 @@
 // the gfx950 buffer_load ... lds DMA (8 rows of 128 bytes per instruction,
 // XOR-swizzled 16-byte chunks); only the wave that fills a ring reads it, so
 // the K loop has no barrier, and the ring is as deep as the LDS allows.
-// The partial tiles meet in LDS and are added in K order.
+// The partial tiles meet in LDS and are added in K order.  A wave adds its quarter up in
+// two chains, so that the sum is no further from 64 bits than with 8 K partitions in
+// router_gemm.hip (relative error, E = 64, H = 8192, T = 128: one chain a wave 2.73e-7,
+// two 1.89e-7, 8 partitions 1.92e-7; E = 64, H = 4096 1.92e-7, 1.36e-7, 1.40e-7).
 // The blocks of one row tile are 8 apart in the grid: one XCD, whose L2 serves
 // the row tile's x to all of them.
 //
@@ -38,6 +41,8 @@ namespace moe {
 namespace wk {
 // word 3 of a gfx9 raw buffer resource (32-bit data format, no swizzle)
 constexpr int kRsrcW3 = 0x00020000;
+// fp32 chains that a logit's K is added up in, as many as K partitions in router_gemm.hip
+constexpr int kChains = 8;
 // an offset past every resource here: such a load writes zeros and moves nothing
 constexpr int kPast = 0x7f000000;
 __device__ __forceinline__ int swz(int r) { return (r >> 1) & 7; }
@@ -66,6 +71,7 @@ __global__ __launch_bounds__(64 * NW) void router_wk_kernel(const __bf16* __rest
   constexpr int RING_B = NW * NS * STAGE_B, PART_B = NW * BM * LD * 4;
   __shared__ __attribute__((aligned(1024))) char lds[RING_B > PART_B ? RING_B : PART_B];
   static_assert(sizeof(lds) <= 160 * 1024, "LDS");
+  static_assert(kChains == NW || kChains == 2 * NW, "chains");
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -115,18 +121,18 @@ __global__ __launch_bounds__(64 * NW) void router_wk_kernel(const __bf16* __rest
     }
   };
 
-  f32x4 acc[NP][FM][FN];
+  f32x4 acc[NP][FM][FN], tot[NP][FM][FN];  // tot: the chain before this one
 #pragma unroll
   for (int p = 0; p < NP; ++p)
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int j = 0; j < FN; ++j) acc[p][i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < FN; ++j) acc[p][i][j] = tot[p][i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int st = 0; st < NS - 1; ++st) issue(st, st);
   const int fr = lane & 15, fc = lane >> 4;
   int slot = 0;
-  for (int u = 0; u < n; ++u) {
+  auto step = [&](int u) __attribute__((always_inline)) {
     // stage u landed once at most the NS-2 later stages are outstanding; the
     // slot refilled now held step u-1, whose reads its MFMAs have consumed
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * NQ) : "memory");
@@ -168,7 +174,23 @@ __global__ __launch_bounds__(64 * NW) void router_wk_kernel(const __bf16* __rest
         }
       }
     }
+  };
+  // An fp32 chain's error grows with its length: a wave with a quarter of K adds it up in
+  // two (kChains).
+  int u = 0;
+  if constexpr (kChains > NW) {
+    for (; u < n / 2; ++u) step(u);
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          tot[p][i][j] = acc[p][i][j];
+          acc[p][i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        }
   }
+  for (; u < n; ++u) step(u);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the loads past u1 have landed
   __syncthreads();  // every ring is read: the partial tiles may overwrite them
   float* const part = reinterpret_cast<float*>(lds);
@@ -185,7 +207,8 @@ __global__ __launch_bounds__(64 * NW) void router_wk_kernel(const __bf16* __rest
       for (int j = 0; j < FN; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          part[(wave * BM + i * 16 + fc * 4 + r) * LD + j * 16 + fr] = acc[p][i][j][r];
+          part[(wave * BM + i * 16 + fc * 4 + r) * LD + j * 16 + fr] =
+              tot[p][i][j][r] + acc[p][i][j][r];
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < PER; ++q) {

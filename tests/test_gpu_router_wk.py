@@ -143,3 +143,35 @@ def test_uneven_k_partitions(cuda, E, H, T, fp32):
     assert_logits(logits, x, w, fp32)
     i2, w2, c2 = M.topk(logits, None, 8, RouteCfg())
     assert torch.equal(ids, i2) and torch.equal(wts, w2) and torch.equal(counts, c2)
+
+
+def chained(x, w, parts):
+    """x . w^T as the matrix instruction adds it, a rounding to fp32 every 8 products, in
+    `parts` chains of equal length that are then added."""
+    x, w, U = x.double(), w.double(), x.shape[1] // 64
+    total = None
+    for z in range(parts):
+        acc = None
+        for k in range(z * U // parts * 64, (z + 1) * U // parts * 64, 8):
+            p = x[:, k:k + 8] @ w[:, k:k + 8].t()
+            acc = (p if acc is None else acc.double() + p).float()
+        total = acc if total is None else total + acc
+    return total
+
+
+@pytest.mark.parametrize("E,H,T,parts", [
+    (64, 4096, 128, 8), (64, 8192, 700, 8), (32, 1024, 2500, 8), (256, 2048, 1100, 8),  # waves
+    (256, 4096, 8000, 4), (256, 1024, 12000, 4), (128, 1024, 12000, 2),  # whole-K tiles
+    (256, 8192, 4904, 8), (128, 8192, 3000, 8)])  # fewer partitions than that
+def test_error_of_the_sum(cuda, E, H, T, parts):
+    """No further from the float64 product than K in as many fp32 chains as the general
+    GEMM has partitions at this size.  3%: the two errors are norms over 8192 values and
+    more, each within 1 / sqrt(2 * 8192) = 0.8% of its expectation."""
+    x, w = inputs(T, H, E, 7, cuda)
+    w = w.bfloat16()
+    logits = M.route(x, w, None, 8, RouteCfg())[0]
+    ref = x.double() @ w.double().t()
+    err = float((logits.double() - ref).norm() / ref.norm())
+    of_chains = float((chained(x, w, parts).double() - ref).norm() / ref.norm())
+    print("sum E=%d H=%d T=%d: %.3g, %d chains %.3g" % (E, H, T, err, parts, of_chains), flush=True)
+    assert err <= 1.03 * of_chains
