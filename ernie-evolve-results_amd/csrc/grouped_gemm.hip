@@ -357,8 +357,12 @@ __device__ constexpr int sc_at(int buf, int x) { return 8 * kHalf + (buf * 2 + x
 // bf16 / int8 tiles of at most 128 rows: stages of B0, B1 and up to 128 rows of A
 constexpr int kStages = 3, kRunMax = 2;
 template <GgType TY, bool SHORT>
-constexpr int kLds = TY == kFp8 ? 8 * kHalf + 8192 : SHORT ? kStages * 3 * kHalf : 8 * kHalf;
-static_assert(kStages * 3 >= 8, "LDS map");
+constexpr int kLds = TY == kFp8 ? 8 * kHalf + 8192
+                   : SHORT      ? kStages * 3 * kHalf
+                                : 8 * kHalf + (TY == kInt8 ? 2048 : 0);
+// int8: the tile's row scales and column scales, past the operands
+constexpr int kScales = 8 * kHalf;
+static_assert(kStages * 3 * kHalf >= kScales + 2048, "LDS map");
 
 template <int N>
 __device__ __forceinline__ void wait_vm() {
@@ -741,6 +745,25 @@ __global__ __launch_bounds__(512) void grouped_gemm_kernel(
   }
   {
     set_b(nt);
+    if constexpr (I8) {
+      // The scales land under the K loop: 256 row scales (waves 0 .. 3), then the 256
+      // column scales in B row order.  As loads at the epilogue's start (36 a lane, behind
+      // the row indexes) nothing hid them, and short K was slower than with 128 x 512 tiles
+      // (256 rows an expert on average, weights N x K, us, 128 x 512 tiles / loads there /
+      // this: 64 experts 1024 x 512 30.4 / 31.4 / 27.0, 200 rows 20.1 / 20.5 / 18.2;
+      // 64 experts SwiGLU 512 x 1024 43.4 / 43.0 / 38.1; 32 experts SwiGLU 3584 x 8192
+      // 677 / 575 / 562).
+      const int i = (wave & 3) * 64 + lane;
+      const float* src;
+      if (wave < 4) {
+        const int row = min(r0 + i, rlast);
+        src = ident ? ex.ident + (row - gs) : ex.a + (ex.a_idx ? ex.a_idx[row] : row);
+      } else {
+        const int col = SWIGLU ? nt * 128 + (i & 127) : nt * 256 + i;
+        src = (SWIGLU && i >= 128 ? ex.w1 : ex.w0) + (long long)g * N + min(col, N - 1);
+      }
+      dma4((const char*)src, lds + kScales + wave * 256);
+    }
     issue_b(0, 0);
     issue_a(0, 0);
     if constexpr (F8) issue_s(0, 0);
@@ -832,34 +855,23 @@ __global__ __launch_bounds__(512) void grouped_gemm_kernel(
 
   // ---- epilogue: element e of a 16 x 16 block is row fc*4 + e, column fr.
   // SwiGLU: B half 0 is the gate, half 1 the up product of the same columns.
-  // int8: value = float(acc) * (row scale * column scale); all scales are
-  // loaded before the first store (a load issued after a store waits for it).
+  // int8: value = float(acc) * (row scale * column scale).
   constexpr int OUTC = SWIGLU ? 128 : 256, NY = SWIGLU ? 1 : 2;
   auto colof = [&](int y, int j) { return y * 128 + wn * 32 + j * 16 + fr; };
   auto rowof = [&](int x, int i, int e) { return x * 128 + wm * 64 + i * 16 + fc * 4 + e; };
-  float cs[2][2], rs[2][4][4];
+  float cs[2][2];
+  f32x4 rs[2][4];
+  if constexpr (I8) {
+    const float* sc = reinterpret_cast<const float*>(lds + kScales);
 #pragma unroll
-  for (int y = 0; y < 2; ++y)
+    for (int y = 0; y < 2; ++y)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      cs[y][j] = 1.0f;
-      if constexpr (I8) {
-        const int col = nt * OUTC + colof(SWIGLU ? 0 : y, j);
-        if (col < N) cs[y][j] = (SWIGLU && y ? ex.w1 : ex.w0)[(long long)g * N + col];
-      }
-    }
+      for (int j = 0; j < 2; ++j) cs[y][j] = sc[256 + colof(y, j)];
 #pragma unroll
-  for (int x = 0; x < 2; ++x)
+    for (int x = 0; x < 2; ++x)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        rs[x][i][e] = 1.0f;
-        if constexpr (I8) {
-          const int row = min(r0 + rowof(x, i, e), rlast);
-          rs[x][i][e] = ident ? ex.ident[row - gs] : ex.a[ex.a_idx ? ex.a_idx[row] : row];
-        }
-      }
+      for (int i = 0; i < 4; ++i) rs[x][i] = *reinterpret_cast<const f32x4*>(sc + rowof(x, i, 0));
+  }
   auto product = [&](int x, int y, int i, int j, int e) -> float {
     if constexpr (I8) return (float)acc[x][y][i][j][e] * (rs[x][i][e] * cs[y][j]);
     else return acc[x][y][i][j][e];

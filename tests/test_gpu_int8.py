@@ -135,6 +135,24 @@ def test_grouped_gemm_i8_identity_groups(cuda):
     assert torch.equal(out.cpu(), ref)
 
 
+@pytest.mark.parametrize("N", [131, 512])
+@pytest.mark.parametrize("K", [128, 384])
+def test_grouped_gemm_i8_scales_of_large_tiles(cuda, N, K):
+    """Groups of several row tiles, the last one partial, some of them identity groups, one
+    and three K steps, a partial column tile: each row and column its own scale."""
+    sizes, T = [300, 257, 300, 129, 600], 300
+    a, w, rs, idx, ws = make_i8(sizes, N, K, seed=N + K)
+    rng = np.random.default_rng(K)
+    ident = rng.integers(-127, 128, size=(T, K)).astype(np.int8)
+    ids = (rng.random(T) * 0.01 + 0.001).astype(np.float32)
+    t = lambda v: torch.from_numpy(v).to(cuda)
+    out = M.grouped_gemm_i8(t(a), t(rs), t(w), t(ws), inclusive(sizes, cuda), ident_a=t(ident),
+                            ident_scales=t(ids), ident_m=T)
+    ref = bf16(O.grouped_gemm_i8(a, rs, w, ws, np.cumsum(sizes), ident_a=ident,
+                                 ident_scales=ids, ident_m=T))
+    assert torch.equal(out.cpu(), ref)
+
+
 @pytest.mark.parametrize("sizes,N,K", [([3, 150, 0, 77], 384, 512), ([900, 1200], 256, 640)])
 def test_grouped_swiglu_i8(cuda, sizes, N, K):
     rng = np.random.default_rng(len(sizes) * 31 + K)
