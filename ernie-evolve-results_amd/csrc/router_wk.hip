@@ -258,9 +258,8 @@ struct Tile {
 // block's waves on one tile), for batches of several rounds.
 const Tile kTiles[] = {
     {16, 16, launch_wk<16, 16, 4, 4, false>}, {32, 16, launch_wk<32, 16, 4, 3, false>},
-    {16, 32, launch_wk<16, 32, 4, 3, false>}, {48, 16, launch_wk<48, 16, 4, 3, false>},
-    {32, 32, launch_wk<32, 32, 4, 3, false>}, {48, 32, launch_wk<48, 32, 4, 3, false>},
-    {64, 32, launch_wk<64, 32, 4, 3, false>}, {32, 64, launch_wk<32, 64, 4, 3, false>},
+    {48, 16, launch_wk<48, 16, 4, 3, false>}, {32, 32, launch_wk<32, 32, 4, 3, false>},
+    {48, 32, launch_wk<48, 32, 4, 3, false>}, {64, 32, launch_wk<64, 32, 4, 3, false>},
     {48, 64, launch_wk<48, 64, 4, 2, false>}, {64, 64, launch_wk<64, 64, 4, 2, false>},
     {80, 64, launch_wk<80, 64, 4, 2, false>}, {128, 64, launch_router_gemm_128x64},
     {128, 128, launch_router_gemm_128x128}};
