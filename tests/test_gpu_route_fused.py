@@ -1,13 +1,15 @@
-"""The fused router GEMM + scoring kernel (E = 256, H = 7168 with 128-token
-tiles; E = 128, H = 2048 with 64-token tiles) against the
-two-kernel path it replaces (moe_router_gemm, then moe_topk on the logits it
-wrote) and against the oracle on the kernel's own logits.
+"""The route at the shapes of the fused router GEMM + scoring kernel (E = 256, H = 7168
+with 128-token tiles; E = 128, H = 2048 with 64-token tiles) against the two calls
+moe_router_gemm, then moe_topk on the logits it wrote, and against the oracle on the
+route's own logits.
 
-The fused kernel accumulates K in the same order as the standalone GEMM, so
-its logits are bit-identical to it, and selection on identical logits is
-bit-identical (ids, weights, counts).  Cases: token counts that are not a
-multiple of the 128-token tile (1, 77, 129, 1000, 4133), one full tile,
-every scoring rule the fused path takes, k = 8 (compile-time) and k = 5
+The fused kernel takes the batches above 16384 (10240) tokens.  It accumulates K in the
+same order as the standalone GEMM, so its logits are bit-identical to it, and selection
+on identical logits is bit-identical (ids, weights, counts).  Smaller batches run the GEMM
+with K split over the waves of a block, in moe_router_gemm too, and the scoring kernel:
+there the comparison with the oracle is the test.  Cases: token counts that are not a
+multiple of a tile, one full tile, the first batch of the fused kernel and others that
+end inside its tiles, every scoring rule it takes, k = 8 (compile-time) and k = 5
 (runtime), bias present and absent.  Needs an MI355X."""
 import ctypes
 
@@ -22,7 +24,10 @@ from oracle import moe_oracle as O
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(256, 7168), (128, 2048)]  # (E, H) the fused kernel takes
+# (E, H, T of the first batch that the fused kernel takes)
+SHAPES = [(256, 7168, 16385), (128, 2048, 10241)]
+CASES = [(E, H, T) for E, H, first in SHAPES
+         for T in (1, 77, 128, 129, 1000, 4133, first, first + 76, first + 131)]
 
 CFGS = {
     "sigmoid_group": RouteCfg(SCORING_SIGMOID_GROUP, True, 8, 4, 2.5),
@@ -42,9 +47,8 @@ def two_kernel_route(x, w, bias, k, cfg):
     return logits, ids, wts, counts
 
 
-@pytest.mark.parametrize("T", [1, 77, 128, 129, 1000, 4133])
+@pytest.mark.parametrize("E,H,T", CASES)
 @pytest.mark.parametrize("rule", ["sigmoid_group", "softmax", "softmax_bias"])
-@pytest.mark.parametrize("E,H", SHAPES)
 def test_fused_route_matches_two_kernel_path(cuda, T, rule, E, H):
     cfg = CFGS[rule]
     if rule == "sigmoid_group" and E == 128:
@@ -75,11 +79,12 @@ def test_fused_route_matches_two_kernel_path(cuda, T, rule, E, H):
     assert np.all(np.abs(got - ow) <= 1e-5 * np.abs(ow) + 1e-30)
 
 
-@pytest.mark.parametrize("E,H", SHAPES)
-def test_fused_route_workspace_and_repeat(cuda, E, H):
-    """Two calls in a row with the same workspace (rewritten by every call)
-    give the same bits; the workspace is checked on the host."""
-    T, k = 300, 8
+@pytest.mark.parametrize("E,H,T", SHAPES)
+def test_fused_route_workspace_and_repeat(cuda, E, H, T):
+    """Calls with one weight, another and the first again in the same workspace (its
+    weight copy is rewritten by every call): each has its own weight's logits, the first
+    and the last the same bits; the workspace is checked on the host."""
+    k = 8
     cfg = CFGS["sigmoid_group"] if E == 256 else CFGS["softmax"]
     g = torch.Generator().manual_seed(11)
     x = torch.randn(T, H, generator=g).bfloat16().to(cuda)
@@ -103,6 +108,9 @@ def test_fused_route_workspace_and_repeat(cuda, E, H):
     torch.cuda.synchronize()
     assert torch.equal(outs[0][0], outs[2][0]) and torch.equal(outs[0][1], outs[2][1])
     assert not torch.equal(outs[0][0], outs[1][0])
+    for (lg, ids, _), ww in zip(outs, (w, w2, w)):
+        lo, ido, _, _ = two_kernel_route(x, ww, bias, k, cfg)
+        assert torch.equal(lg, lo) and torch.equal(ids, ido)
     rc = L.moe_route(M._ptr(x), M._ptr(w), 0, M._ptr(bias), T, H, E, k, ctypes.byref(c),
                      M._ptr(outs[0][0]), M._ptr(outs[0][1]), M._ptr(outs[0][2]), None,
                      M._ptr(ws), nws - 256, M._stream(x))
@@ -111,7 +119,8 @@ def test_fused_route_workspace_and_repeat(cuda, E, H):
 
 @pytest.mark.parametrize("topk_group", [1, 2, 3, 4, 6, 8])
 @pytest.mark.parametrize("k", [8, 6])
-def test_fused_sigmoid_group_ties_and_kept_group_counts(cuda, topk_group, k):
+@pytest.mark.parametrize("T", [300, 16391])
+def test_fused_sigmoid_group_ties_and_kept_group_counts(cuda, T, topk_group, k):
     """E = 256 in 8 groups of 32 (one scoring lane per group, two tokens per
     lane group: with at most 4 kept groups the epilogue ranks only those,
     compacted into the lane group; with more it ranks all 8 lanes).  Router
@@ -119,8 +128,8 @@ def test_fused_sigmoid_group_ties_and_kept_group_counts(cuda, topk_group, k):
     scores tie exactly, inside a group and across groups; ties go to the
     lower expert index.  The fused kernel must select what the one-token
     scoring kernel and the oracle select on the same logits, for 1 to 8
-    kept groups."""
-    E, H, T = 256, 7168, 300
+    kept groups (T = 300: the scoring kernel itself, against the oracle)."""
+    E, H = 256, 7168
     cfg = RouteCfg(SCORING_SIGMOID_GROUP, True, 8, topk_group, 2.5)
     g = torch.Generator().manual_seed(100 + 10 * topk_group + k)
     x = torch.randn(T, H, generator=g).bfloat16()
@@ -131,7 +140,7 @@ def test_fused_sigmoid_group_ties_and_kept_group_counts(cuda, topk_group, k):
     lf, idf, wf, cf = M.route(x, w, bias, k, cfg)
     lo, ido, wo, co = two_kernel_route(x, w, bias, k, cfg)
     torch.cuda.synchronize()
-    print("ties topk_group=%d k=%d" % (topk_group, k), flush=True)
+    print("ties T=%d topk_group=%d k=%d" % (T, topk_group, k), flush=True)
     assert torch.equal(lf, lo)
     # exact ties are present: expert e and e + 37 have equal logits
     assert torch.equal(lf[:, 0], lf[:, 37])

@@ -3,15 +3,16 @@ calls it stands for, moe_route then moe_permute: every output bit-identical
 (logits, ids, weights, gathered bf16 rows or fp8 bytes + scales, row_token,
 pair_row, offsets, counts).
 
-Where the route is the fused kernel and k divides 256 with 256 / k tokens
-fitting its token tile (E = 256: k in {2, 4, 8}; E = 128: k in {4, 8}), the
-fused kernel's epilogue writes the permute's block histograms; on the
-two-kernel route (other shapes, fp32 weights) the scoring kernel writes them
-when k divides 256; the small-E route kernel (E = 8 or 16, H % 256 == 0)
+Where the route is the fused kernel (E = 256, H = 7168 above 16384 tokens, E = 128,
+H = 2048 above 10240) and k divides 256 with 256 / k tokens fitting its token tile
+(E = 256: k in {2, 4, 8}; E = 128: k in {4, 8}), the fused kernel's epilogue writes the
+permute's block histograms; on the two-kernel route (smaller batches, other shapes, fp32
+weights) the scoring kernel writes them when k divides 256; up to 2048 pairs, where the
+permute is one launch, nothing does; the small-E route kernel (E = 8 or 16, H % 256 == 0)
 writes one histogram per 32 tokens, which the index kernel sums per block
 when 256 / k is a multiple of 32 and E x columns <= 8192.  These cases check both handoffs: token counts that end
-inside a block of 256 pairs and inside a route tile (1, 33, 129, 1000,
-4133), k = 5, 3 and (fused) 1 (no handoff), unfused shapes from E = 8 to
+inside a block of 256 pairs and inside a route tile (33, 129, 1000, 4133, 10241,
+16391), k = 5, 3 and (fused) 1 (no handoff), unfused shapes from E = 8 to
 E = 256, C2's split-K GEMM and fp32 weights (the hi/lo split route of the
 reference's run() shape).  Needs an MI355X."""
 import ctypes
@@ -110,15 +111,25 @@ CASES = [
     (256, 7168, 8, 129, True, False),
     (256, 7168, 8, 1000, False, True),
     (256, 7168, 8, 4133, False, False),
-    (256, 7168, 4, 77, False, False),      # 64-token blocks
-    (256, 7168, 2, 300, True, False),      # 128-token blocks = one tile
-    (256, 7168, 5, 333, False, False),     # no handoff: 256 % 5 != 0
-    (256, 7168, 1, 129, False, False),     # no handoff: 256-token blocks > tile
+    (256, 7168, 4, 77, False, False),      # few pairs: one launch
+    (256, 7168, 2, 300, True, False),
+    (256, 7168, 5, 333, False, False),
+    (256, 7168, 1, 129, False, False),
+    # the fused kernel's histograms
+    (256, 7168, 8, 16391, False, False),   # 32-token blocks, four in a tile
+    (256, 7168, 8, 16500, True, False),
+    (256, 7168, 4, 16391, False, True),    # 64-token blocks
+    (256, 7168, 2, 16391, True, True),     # 128-token blocks = one tile
+    (256, 7168, 5, 16391, False, True),    # no handoff: 256 % 5 != 0
+    (256, 7168, 1, 16391, False, True),    # no handoff: 256-token blocks > tile
     (128, 2048, 8, 1, False, False),
     (128, 2048, 8, 65, False, False),
     (128, 2048, 8, 4133, True, False),
-    (128, 2048, 4, 1000, False, False),    # 64-token blocks = one tile
-    (128, 2048, 2, 200, False, False),     # no handoff: 128-token blocks > tile
+    (128, 2048, 4, 1000, False, False),
+    (128, 2048, 2, 200, False, False),
+    (128, 2048, 8, 10241, False, False),   # fused: 32-token blocks, two in a tile
+    (128, 2048, 4, 10300, True, False),    # 64-token blocks = one tile
+    (128, 2048, 2, 10300, False, True),    # no handoff: 128-token blocks > tile
     (64, 1024, 8, 1000, False, False),     # unfused route: the scoring kernel's handoff
     (64, 8192, 8, 1571, False, True),      # fp32 weights (hi/lo split): the run() shape
     (8, 4096, 2, 8192, False, False),      # C2's shape: the small-E route, 4 columns per block

@@ -131,12 +131,32 @@ def test_fused_kernel_block_histograms(cuda, E, H, T, k):
         assert torch.equal(getattr(plan, name), p[name]), name
 
 
-@pytest.mark.parametrize("E,H,T,fp32", [(64, 8192, 4133, True), (64, 8192, 4904, True),
-                                        (256, 8192, 4133, False), (256, 8256, 5000, False),
-                                        (128, 4160, 6001, True), (256, 1088, 1100, True)])
-def test_uneven_k_partitions(cuda, E, H, T, fp32):
-    """K split over blocks into 3 to 7 parts of unequal length, the partial sums
-    added by the scoring kernel."""
+# (E, H, T, fp32, parts): shapes outside the rule whose K is split over blocks into parts of
+# unequal length, and three whose H is an odd number of 64s and stays whole
+PARTS = [(64, 8192, 4133, True, 3), (64, 8192, 4904, True, 3), (256, 8192, 4133, False, 7),
+         (128, 4608, 6001, True, 5), (256, 1024, 2100, True, 7), (256, 8704, 5000, False, 6),
+         (256, 8256, 5000, False, 1), (128, 4160, 6001, True, 1), (256, 1088, 1100, True, 1)]
+
+
+def partitions(T, H, N):
+    """The general GEMM's: doubled up to 8 while its tiles leave CUs idle and H divides
+    (the workspace's count), then the largest whose rounds of 256 blocks are shortest."""
+    bm, bn = (256, 128) if N >= 256 else (64, N)
+    blocks, most = -(-T // bm) * -(-N // bn), 1
+    while blocks * most < 256 and most < 8 and H % (128 * most) == 0:
+        most *= 2
+    return most, min(range(most, 0, -1), key=lambda p: -(-blocks * p // 256) / p)
+
+
+@pytest.mark.parametrize("E,H,T,fp32,parts", PARTS)
+def test_uneven_k_partitions(cuda, E, H, T, fp32, parts):
+    """K split over blocks, the partial sums added by the scoring kernel."""
+    N = 2 * E if fp32 else E
+    most, run = partitions(T, H, N)
+    assert run == parts and (parts == 1 or H // 64 % parts)
+    sums = T * most * N * 4 if most * N > E else 0
+    assert M.lib().moe_route_workspace_bytes(T, H, E, int(fp32)) == \
+        (N * H * 2 if fp32 else 0) + (sums + 255) // 256 * 256
     x, w = inputs(T, H, E, T + E, cuda)
     w = w if fp32 else w.bfloat16()
     logits, ids, wts, counts = M.route(x, w, None, 8, RouteCfg())
