@@ -20,10 +20,10 @@
 // the row tile's x to all of them.
 //
 // Measured (MI355X; route = this GEMM + the scoring kernel, graph replay, us,
-// the path it replaced first): E = 256, H = 7168: T = 4 91 / 13, 128 91 / 15,
-// 1024 92 / 22, 4096 98 / 44, 8192 99 / 67, 16384 105 / 102; E = 128,
-// H = 2048: T = 128 19 / 9.5, 4096 20 / 15; E = 64, H = 4096: T = 128
-// 11.5 / 8.9.  GEMM alone at E = 256, H = 7168, T = 16: fragments loaded
+// the path it replaced first): E = 256, H = 7168: T = 16 88 / 11.2, 128 91 / 11.6,
+// 1024 92 / 18.9, 4904 92 / 35.8, 8000 92 / 53.9, 16000 93 / 83.8; E = 128,
+// H = 2048: T = 128 17.8 / 8.5, 4904 18.3 / 14.9; E = 64, H = 4096: T = 128
+// 11.0 / 8.0.  GEMM alone at E = 256, H = 7168, T = 16: fragments loaded
 // straight into registers (16 rows x 64 bytes per load instruction, so every
 // four lanes touch four lines) 15.4 us, this ring 6.5; 8 waves x 2 stages 7.0,
 // 4 waves x 3 stages 7.7.
@@ -32,8 +32,8 @@
 // k into hi = bf16(w) and lo = bf16(w - hi) (the reference's wsplit_kernel,
 // K:1786-1824); a logit is (sum of hi) + (sum of lo), each in K order.  That
 // saves the split's launch, its [2E, H] copy and the partial sums: E = 64,
-// H = 8192 T = 128 20.5 / 13.5, T = 3000 32.7 / 28.9; E = 256, H = 1024
-// T = 128 20.7 / 11.5.
+// H = 8192 T = 128 19.4 / 12.6, T = 3000 26.3 / 22.0; E = 256, H = 1024
+// T = 128 16.8 / 8.9.
 #include "moe_common.h"
 
 namespace moe {
@@ -293,26 +293,34 @@ static const Tile* pick(int T, int E, bool wf32) {
 
 // Where it takes over (route times in us, the other path / this one):
 //   E = 256, H = 7168 and E = 128, H = 2048 (the fused kernel's shapes): while
-//     the fused kernel's tiles fill under ~2/3 of the CUs: T = 16384 105 / 102,
-//     24000 116 / 188; T = 10000 22.4 / 21.6, 12000 24.8 / 29.6.
+//     the fused kernel's tiles fill at most half (5/8) of the CUs: T = 16000 94 / 89,
+//     18000 101 / 143; T = 10000 21.6 / 20.3, 12000 22.3 / 23.1.
 //   elsewhere, against K split over blocks with the partial sums added by the
-//     scoring kernel: that path moves fewer operand bytes (larger tiles) but
-//     writes and reads the partials, so it wins for long rows and many tokens:
-//     E = 256, H = 4096 T = 4500 32 / 25, 6000 31 / 34, 7000 49 / 35, 10100 40 / 47,
-//     12200 53 / 50, 32768 91 / 120; H = 2048 T = 12200 44 / 32; E = 64, H = 8192
-//     T = 900 13.8 / 12.5, 2300 17.3 / 17.5, 2800 18.2 / 18.0.
+//     scoring kernel.  That path moves fewer operand bytes (larger tiles) but
+//     writes and reads the partials; either is ahead as its tiles fill whole rounds:
+//     E = 256, H = 4096 T = 4500 33.3 / 27.1, 6000 32.7 / 36.7, 7000 51.8 / 37.4,
+//     10100 43.1 / 49.2, 12200 58.5 / 48.9; E = 64, H = 8192 T = 900 13.8 / 11.8,
+//     2300 17.6 / 17.5.  The lines lie where the two met when the partitions were fewer
+//     and the chains longer; past them this kernel is still as fast or faster up to
+//     16000 tokens at H <= 4096 (E = 256, H = 4096 T = 13000 67.8 / 52.3, H = 1024
+//     T = 16000 47.2 / 28.8; E = 64, H = 4096 T = 14000 27.7 / 26.8), and at H = 8192 up
+//     to 3500 (E = 256 38.7 / 32.6; E = 64 19.7 / 18.6), not at E = 256,
+//     H = 4096 T = 32768 (106 / 122).
 //   E = 128 above 8192 tokens, where that path has one tile of 64 tokens and all
 //     experts per 64 tokens and no K split: the 80 x 64 tiles up to 10240 (H = 4096
-//     T = 9000 32 / 26).  From there the tiles are 128 x 64, above 16384 128 x 128.
-//     They have the same operand bytes per CU (up to 16384 tokens) and lose while x
-//     stays in the 256 MB memory-side cache, except where H is short (H = 1024
-//     T = 12200 20.8 / 17.8, 25000 23.3 / 23.9; H = 4096 T = 12200 33.5 / 34.9, 22000
-//     47 / 49; H = 8192 T = 11000 49 / 57), and win beyond (H = 8192 T = 15000 74 / 61,
-//     18000 125 / 93; H = 7168 T = 32768 140 / 115) unless the last of the 128-token
-//     rounds is nearly empty (H = 8192 T = 45000 216 / 231).
-//   fp32 weights: E = 64, H = 8192 T = 3000 32.7 / 28.9, 4096 34.9 / 42.0;
-//     E = 256, H = 4096 T = 700 30 / 19, 4096 42 / 61; E = 32, H = 4096
-//     T = 6000 22.9 / 20.0, 8192 27.9 / 29.1.
+//     T = 9000 31.5 / 25.9).  From there the tiles are 128 x 64, above 16384 128 x 128.
+//     They have the same operand bytes per CU (up to 16384 tokens) and lose or tie while
+//     x stays in the 256 MB memory-side cache, except where H is short (H = 1024
+//     T = 12200 20.5 / 17.4, 25000 25.5 / 25.1; H = 4096 T = 12200 32.9 / 34.4, 22000
+//     49 / 47; H = 8192 T = 11000 49 / 56), and win beyond (H = 8192 T = 15000 76 / 58,
+//     18000 124 / 98; H = 7168 T = 32768 138 / 115) unless the last of the 128-token
+//     rounds is nearly empty (H = 8192 T = 45000 215 / 225).
+//   fp32 weights, whose rows count twice: E = 64, H = 8192 T = 3070 25.7 / 21.7, 4000
+//     28.2 / 30.7; E = 256, H = 4096 T = 700 27.0 / 16.3, 890 27.8 / 21.7; E = 32,
+//     H = 4096 T = 6000 19.4 / 15.4, 7100 20.0 / 20.3, 8192 19.7 / 20.6.  At E >= 128 and
+//     at H <= 1024 this kernel is ahead past the line too (E = 256, H = 4096 T = 1200
+//     30.2 / 24.8; E = 128, H = 1024 T = 2600 24.9 / 14.0; E = 64, H = 512 T = 6000
+//     17.3 / 11.8).
 bool router_wk_use(int T, int H, int E, bool wf32) {
   if (T < 1 || E < 32 || H % 64 != 0 || H > 32768) return false;
   if (wf32) return (long long)T * E <= (H <= 4096 ? 229376 : 196608);

@@ -73,15 +73,18 @@ int moe_version(void);
 const char* moe_last_error_string(void);
 
 /* Workspace bytes moe_route needs (the K:4197-4268 arena, caller-owned).
- * Non-zero only when
+ * The sum of what the general path of the shape uses:
  *   - w_dtype is FP32: the hi/lo split weight [2E,H] bf16, plus
  *   - the GEMM writes more than one partial logit block per row, i.e. FP32
- *     weights (hi and lo halves) or a K split (ksplit > 1, chosen when the
- *     row x expert tiles alone leave the chip's 256 CUs idle, e.g. small T):
- *     [T, parts*E] fp32 partial sums.
+ *     weights (hi and lo halves) or a K split (chosen when the row x expert
+ *     tiles alone leave the chip's 256 CUs idle, e.g. small T): [T, parts*E]
+ *     fp32 partial sums.
  *   - E = 256, H = 7168 or E = 128, H = 2048 with bf16 weights: for large T the
  *     GEMM and the scoring run as one kernel that reads a fragment-major copy
  *     of the weight, E*H*2 bytes (3.5 MiB / 512 KiB), rewritten by every call.
+ * Batches of E >= 32 that take the GEMM with K split over the waves of a block
+ * (moe_route) leave it unused, and the size stays as it is: it depends on the
+ * arguments alone, not on which kernel is the faster one for them.
  * E = 8 or 16 with bf16 weights and H % 256 == 0 (the Mixtral shape): zero;
  * one kernel does the GEMM, with K split across the four waves of a block,
  * and the scoring (E = 8 with FP32 weights too: the kernel splits the weight
@@ -91,6 +94,8 @@ size_t moe_route_workspace_bytes(int T, int H, int E, int w_dtype);
 
 /* Stage 1: router GEMM, logits[T,E] fp32 = x[T,H] bf16 . w[E,H]^T bf16, fp32
  * accumulate on MFMA.  Replaces the cublasGemmEx call K:4327-4339.
+ * How K is divided, and so the order of the fp32 sums, depends on T: the same
+ * token's logits may differ in their last bits between batch sizes.
  * Needs H % 64 == 0 and E in {8,16,32,64,128,256}. */
 int moe_router_gemm(const void* x, const void* w, int T, int H, int E, float* logits,
                     void* stream);
@@ -108,11 +113,14 @@ int moe_topk(const float* logits, const float* bias, int T, int E, int k,
  * w_dtype BF16: w is [E,H] bf16.  w_dtype FP32: w is [E,H] fp32 and is split
  * into bf16 hi/lo on the device (wsplit_kernel K:1786-1824) so the bf16 GEMM
  * yields fp32-accurate logits.  logits [T,E] fp32 (the reference's
- * router_logits output), counts may be NULL.  With bf16 weights at E = 256,
- * H = 7168 (T > 16384) or E = 128, H = 2048 (T > 10240) the GEMM and the
- * scoring are one kernel; smaller batches split K over the waves of a block
- * instead (unless a group-limited rule's groups are not multiples of 32 experts at
- * E = 256, 16 at E = 128: then the two-kernel path, same results). */
+ * router_logits output; last bits by T as in moe_router_gemm), counts may be
+ * NULL.  With bf16 weights at E = 256, H = 7168 (T > 16384) or E = 128, H = 2048
+ * (T > 10240) the GEMM and the scoring are one kernel (unless a group-limited
+ * rule's groups are not multiples of 32 experts at E = 256, 16 at E = 128: then
+ * two).  Smaller batches there, and the batches of other shapes
+ * with E >= 32 that would leave much of the chip idle, take a GEMM with K split
+ * over the waves of a block, or from about 1.3 million logits on (T * E) one of
+ * 128-token tiles over all of K, and then the scoring kernel. */
 int moe_route(const void* x, const void* w, int w_dtype, const float* bias, int T, int H,
               int E, int k, const moe_route_cfg* cfg, float* logits, int32_t* topk_ids,
               float* topk_w, int32_t* counts, void* ws, size_t ws_bytes, void* stream);
