@@ -30,6 +30,7 @@
 // Smaller N use smaller row tiles (and split-K when even those leave the
 // chip idle): there the router weight is small and the GEMM is an x stream.
 #include "moe_common.h"
+#include <type_traits>
 
 namespace moe {
 
@@ -132,7 +133,8 @@ __global__ __launch_bounds__(64 * WM * WN) void router_gemm_dma_kernel(
   for (int st = 0; st < NS - 1; ++st)
     if (st < KT) issue(st, st);
   const int fr = lane & 15, fc = lane >> 4;
-  auto step = [&](int kt) __attribute__((always_inline)) {
+  // FIRST: of a chain, from a constant zero instead of cleared accumulators
+  auto step = [&]<bool FIRST>(std::bool_constant<FIRST>, int kt) __attribute__((always_inline)) {
     // This wave's loads of stage kt are done once at most (NS-2) later
     // stages are outstanding; the barrier then publishes every wave's
     // loads and retires the reads of the buffer reloaded next.
@@ -159,21 +161,22 @@ __global__ __launch_bounds__(64 * WM * WN) void router_gemm_dma_kernel(
       for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              a[i], b[j], FIRST && kk == 0 ? (f32x4){0.f, 0.f, 0.f, 0.f} : acc[i][j], 0, 0, 0);
     }
   };
   if constexpr (FOLD) {
     for (int kt = 0; kt < KT;) {
       const int end = min(kt + fold, KT);
-      for (; kt < end; ++kt) step(kt);
+      step(std::true_type{}, kt++);
+      for (; kt < end; ++kt) step(std::false_type{}, kt);
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) tot[i][j] += acc[i][j];
-      zero(acc);
     }
   } else {
-    for (int kt = 0; kt < KT; ++kt) step(kt);
+    for (int kt = 0; kt < KT; ++kt) step(std::false_type{}, kt);
   }
 
   // partial z of the split-K writes columns [z*N, (z+1)*N) of a row of ldo floats

@@ -35,6 +35,7 @@
 // H = 8192 T = 128 19.4 / 12.6, T = 3000 26.3 / 22.0; E = 256, H = 1024
 // T = 128 16.8 / 8.9.
 #include "moe_common.h"
+#include <type_traits>
 
 namespace moe {
 
@@ -123,16 +124,13 @@ __global__ __launch_bounds__(64 * NW) void router_wk_kernel(const __bf16* __rest
 
   f32x4 acc[NP][FM][FN], tot[NP][FM][FN];  // tot: the chain before this one
 #pragma unroll
-  for (int p = 0; p < NP; ++p)
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j) acc[p][i][j] = tot[p][i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
   for (int st = 0; st < NS - 1; ++st) issue(st, st);
   const int fr = lane & 15, fc = lane >> 4;
   int slot = 0;
-  auto step = [&](int u) __attribute__((always_inline)) {
+  // FIRST: of a chain, from a constant zero instead of cleared accumulators (route at
+  // E = 128, H = 512, T = 8000: one chain a wave 12.7 us, two 13.2, two from the constant 12.6)
+  auto step = [&]<bool FIRST>(std::bool_constant<FIRST>, int u) __attribute__((always_inline)) {
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     // stage u landed once at most the NS-2 later stages are outstanding; the
     // slot refilled now held step u-1, whose reads its MFMAs have consumed
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * NQ) : "memory");
@@ -167,30 +165,43 @@ __global__ __launch_bounds__(64 * NW) void router_wk_kernel(const __bf16* __rest
         }
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
-          acc[0][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], bh, acc[0][i][j], 0, 0, 0);
+          const bool z = FIRST && kk == 0;
+          acc[0][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], bh, z ? zero : acc[0][i][j],
+                                                                 0, 0, 0);
           if constexpr (WF32)
-            acc[1][i][j] =
-                __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], bl, acc[1][i][j], 0, 0, 0);
+            acc[1][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                av[i], bl, z ? zero : acc[1][i][j], 0, 0, 0);
         }
       }
     }
   };
+  int u = 0;
+  auto chain = [&](int end) __attribute__((always_inline)) {
+    if (FM * FN >= 6 && u < end) {  // a third copy of the step costs the small tiles more
+      step(std::true_type{}, u++);
+    } else {
+#pragma unroll
+      for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) acc[p][i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+    for (; u < end; ++u) step(std::false_type{}, u);
+  };
   // An fp32 chain's error grows with its length: a wave with a quarter of K adds it up in
   // two (kChains).
-  int u = 0;
-  if constexpr (kChains > NW) {
-    for (; u < n / 2; ++u) step(u);
+  constexpr bool TWO = kChains > NW;
+  if constexpr (TWO) {
+    chain(n / 2);
 #pragma unroll
     for (int p = 0; p < NP; ++p)
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          tot[p][i][j] = acc[p][i][j];
-          acc[p][i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        }
+        for (int j = 0; j < FN; ++j) tot[p][i][j] = acc[p][i][j];
   }
-  for (; u < n; ++u) step(u);
+  chain(n);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the loads past u1 have landed
   __syncthreads();  // every ring is read: the partial tiles may overwrite them
   float* const part = reinterpret_cast<float*>(lds);
@@ -208,7 +219,7 @@ __global__ __launch_bounds__(64 * NW) void router_wk_kernel(const __bf16* __rest
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           part[(wave * BM + i * 16 + fc * 4 + r) * LD + j * 16 + fr] =
-              tot[p][i][j][r] + acc[p][i][j][r];
+              TWO ? tot[p][i][j][r] + acc[p][i][j][r] : acc[p][i][j][r];
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
