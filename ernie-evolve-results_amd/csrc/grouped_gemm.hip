@@ -31,11 +31,14 @@
 // rows read in one half step are refilled in the next (every wave has waited for
 // its reads before the barrier in between), for the step after next, so a load
 // has three half steps to land and 96 of the 128 KB are in flight or in use.
-// One 256 x 256 tile per CU at 85% MFMA busy (counters, K = 8192; the previous
-// loop, both waves of a SIMD in step and the whole stage refilled at once: 71%).
-// Measured, dense (TFLOP/s or TOP/s, previous loop first): 16384 x 16384 x 8192
-// bf16 1292 / 1489, SwiGLU 1337 / 1501, int8 2623 / 2854; 65536 x 8192 x 3584 bf16
-// 1310 / 1451, int8 2268 / 2455.  The rest is the clock: 1.48 GHz at this load.
+// One 256 x 256 tile per CU.  Measured, dense 16384 x 16384 x 8192, counters and times of
+// the same launches (share of cycles the MFMA units are busy x clock = rate): bf16 86% x
+// 1.56 GHz = 1407 TFLOP/s, SwiGLU 85% x 1.74 = 1545, int8 78% x 1.81 = 2978 TOP/s; the
+// library's bf16 GEMM 89% x 1.59 = 1482.  So 3 points of busy time are the schedule's, and
+// the clock falls as the units are busier; 65536 x 8192 x 3584, where the start and end of
+// a tile weigh more: bf16 79% x 1.77 = 1471, int8 65% x 1.92 = 2631.  The previous loop
+// (both waves of a SIMD in step, the whole stage refilled at once) had bf16 1292, SwiGLU
+// 1337, int8 2623 and, 65536 x 8192 x 3584, 1310 and 2268.
 // The routed experts (64 experts, H = 8192, Ni = 3584, top-8, us): gate+up T = 16
 // 1229 / 1122, 1024 1794 / 1340, 2048 2398 / 2070.  Tried and slower: four half steps
 // of 16 MFMAs (5% instead of 13% gained), s_setprio around the MFMAs (-1%), the DMA issued
@@ -55,7 +58,8 @@
 // 8 experts SwiGLU 2048 x 4096, 16 rows 95 / 49 / 45.  Where the 128 x 512 tiles fill
 // whole rounds of CUs and the weights' rows are a power of two apart they stay 3 .. 6%
 // ahead: bf16 64 experts 4096 x 2048, 16 rows 188 / 206 / 196; SwiGLU 2048 x 4096, 40 rows
-// 363 / 382 / 378; 128 experts 1024 x 512, 100 rows 33 / 40 / 34.4.  Tried: four stages of
+// 363 / 382 / 378; 128 experts 1024 x 512, 100 rows 33 / 40 / 34.4 (at worst 9%: 64 experts
+// 4096 x 2048, 100 rows on average, 210 / - / 230).  Tried: four stages of
 // 40 KB at up to 64 rows (no gain), two steps loaded at a time (-4%), other orders of the
 // tiles over the XCDs (-2 .. -30%), row tiles of equal height instead of a last one with
 // the rest (no gain: 2041 / 2018 .. 2027 at T = 2048).
